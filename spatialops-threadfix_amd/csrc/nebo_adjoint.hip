@@ -221,7 +221,7 @@ extern "C" int nebo_diffusion_forward(const nebo_field_t* phiT, const nebo_field
   hipStream_t s = (hipStream_t)stream;
   const size_t np = field_npts(phi0), bytes = np * sizeof(double);
   double* tmp = nullptr;
-  if ((rc = check_hip(hipMallocAsync((void**)&tmp, 2 * bytes, s), kCtx))) return rc;
+  if ((rc = scratch_alloc((void**)&tmp, 2 * bytes, s, kCtx))) return rc;
   nebo_field_t ck0 = with_values(phi0, ckpt);
   rc = check_hip(hipMemcpyAsync(ckpt, phi0->values, bytes, hipMemcpyDeviceToDevice, s), kCtx);
   if (!rc) rc = fill_ghosts_periodic(&ck0, stream);
@@ -236,7 +236,7 @@ extern "C" int nebo_diffusion_forward(const nebo_field_t* phiT, const nebo_field
   }
   if (!rc && cur != phiT->values)
     rc = check_hip(hipMemcpyAsync(phiT->values, cur, bytes, hipMemcpyDeviceToDevice, s), kCtx);
-  (void)hipFreeAsync(tmp, s);
+  scratch_free(tmp, s);
   return rc;
 }
 

@@ -893,7 +893,7 @@ extern "C" int nebo_masked_assign(const nebo_field_t* lhs, const int32_t* points
   hipStream_t s = (hipStream_t)stream;
   int32_t* pts = nullptr;
   const size_t bytes = sizeof(int32_t) * 3 * (size_t)n_points;
-  if ((rc = check_hip(hipMallocAsync((void**)&pts, bytes, s), ctx))) return rc;
+  if ((rc = scratch_alloc((void**)&pts, bytes, s, ctx))) return rc;
   if ((rc = check_hip(hipMemcpyAsync(pts, points, bytes, hipMemcpyHostToDevice, s), ctx))) return rc;
   dim3 grid((n_points + kBlock - 1) / kBlock);
   const bool one = prog.n_classes == 1, math = uses_math(prog);
@@ -907,7 +907,7 @@ extern "C" int nebo_masked_assign(const nebo_field_t* lhs, const int32_t* points
   else
     hipLaunchKernelGGL((vm_masked_kernel<kVmMaxClasses, true>), grid, dim3(kBlock), 0, s, prog, pts, n_points, out, oX, oXY);
   rc = check_hip(hipGetLastError(), ctx);
-  (void)hipFreeAsync(pts, s);
+  scratch_free(pts, s);
   return rc;
 }
 

@@ -304,7 +304,7 @@ extern "C" int nebo_particle_to_cell(const nebo_field_t* dest, const double* src
   const unsigned blocks = (unsigned)((np + kBlock - 1) / kBlock);
   long* counts = nullptr;
   long* offsets = nullptr;
-  if ((rc = check_hip(hipMallocAsync((void**)&counts, sizeof(long) * 2 * np, s), ctx))) return rc;
+  if ((rc = scratch_alloc((void**)&counts, sizeof(long) * 2 * np, s, ctx))) return rc;
   offsets = counts + np;
   hipLaunchKernelGGL(count_kernel, dim3(blocks), dim3(kBlock), 0, s, counts, g, pc, psize, (long)np, skipped);
   size_t tmp_bytes = 0;
@@ -312,7 +312,7 @@ extern "C" int nebo_particle_to_cell(const nebo_field_t* dest, const double* src
   rc = check_hip(rocprim::exclusive_scan(nullptr, tmp_bytes, counts, offsets, 0L, (size_t)np,
                                          rocprim::plus<long>(), s),
                  ctx);
-  if (!rc) rc = check_hip(hipMallocAsync(&tmp, tmp_bytes, s), ctx);
+  if (!rc) rc = scratch_alloc(&tmp, tmp_bytes, s, ctx);
   if (!rc)
     rc = check_hip(rocprim::exclusive_scan(tmp, tmp_bytes, counts, offsets, 0L, (size_t)np,
                                            rocprim::plus<long>(), s),
@@ -321,11 +321,11 @@ extern "C" int nebo_particle_to_cell(const nebo_field_t* dest, const double* src
   if (!rc) rc = check_hip(hipMemcpyAsync(&last[0], offsets + np - 1, sizeof(long), hipMemcpyDeviceToHost, s), ctx);
   if (!rc) rc = check_hip(hipMemcpyAsync(&last[1], counts + np - 1, sizeof(long), hipMemcpyDeviceToHost, s), ctx);
   if (!rc) rc = check_hip(hipStreamSynchronize(s), ctx);
-  if (tmp) (void)hipFreeAsync(tmp, s);
+  scratch_free(tmp, s);
   tmp = nullptr;
   const long total = last[0] + last[1];
   if (rc || total == 0) {
-    (void)hipFreeAsync(counts, s);
+    scratch_free(counts, s);
     return rc;
   }
   // cells fit 32-bit keys (the field has fewer than 2^31 points, checked above)
@@ -333,8 +333,8 @@ extern "C" int nebo_particle_to_cell(const nebo_field_t* dest, const double* src
   const int cbits = bits_for((uint64_t)npts);
   uint32_t* keys = nullptr;
   double* vals = nullptr;
-  rc = check_hip(hipMallocAsync((void**)&keys, sizeof(uint32_t) * 2 * total, s), ctx);
-  if (!rc) rc = check_hip(hipMallocAsync((void**)&vals, sizeof(double) * 2 * total, s), ctx);
+  rc = scratch_alloc((void**)&keys, sizeof(uint32_t) * 2 * total, s, ctx);
+  if (!rc) rc = scratch_alloc((void**)&vals, sizeof(double) * 2 * total, s, ctx);
   if (!rc) {
     hipLaunchKernelGGL(fill_kernel, dim3(blocks), dim3(kBlock), 0, s, keys, vals, offsets, src, g, pc, psize,
                        (long)np);
@@ -348,7 +348,7 @@ extern "C" int nebo_particle_to_cell(const nebo_field_t* dest, const double* src
     rc = check_hip(rocprim::radix_sort_pairs(nullptr, tmp_bytes, keys, skeys, vals, svals, (size_t)total, 0,
                                              (unsigned)cbits, s),
                    ctx);
-  if (!rc) rc = check_hip(hipMallocAsync(&tmp, tmp_bytes, s), ctx);
+  if (!rc) rc = scratch_alloc(&tmp, tmp_bytes, s, ctx);
   if (!rc)
     rc = check_hip(rocprim::radix_sort_pairs(tmp, tmp_bytes, keys, skeys, vals, svals, (size_t)total, 0,
                                              (unsigned)cbits, s),
@@ -358,10 +358,10 @@ extern "C" int nebo_particle_to_cell(const nebo_field_t* dest, const double* src
                        static_cast<double*>(dest->values), skeys, svals, total);
     rc = check_hip(hipGetLastError(), ctx);
   }
-  if (tmp) (void)hipFreeAsync(tmp, s);
-  if (vals) (void)hipFreeAsync(vals, s);
-  if (keys) (void)hipFreeAsync(keys, s);
-  (void)hipFreeAsync(counts, s);
+  scratch_free(tmp, s);
+  scratch_free(vals, s);
+  scratch_free(keys, s);
+  scratch_free(counts, s);
   return rc;
 }
 

@@ -725,7 +725,7 @@ extern "C" int nebo_transport_forward(const nebo_field_t* phiT, const nebo_field
   hipStream_t st = (hipStream_t)stream;
   const size_t np = field_npts(phi0), bytes = np * sizeof(double);
   double* tmp = nullptr;   // s1, s2 and two ping-pong states
-  if ((rc = check_hip(hipMallocAsync((void**)&tmp, 4 * bytes, st), kCtx))) return rc;
+  if ((rc = scratch_alloc((void**)&tmp, 4 * bytes, st, kCtx))) return rc;
   const Operands o{u, k};
   nebo_field_t ck0 = with_values(phi0, ckpt);
   rc = check_hip(hipMemcpyAsync(ckpt, phi0->values, bytes, hipMemcpyDeviceToDevice, st), kCtx);
@@ -740,7 +740,7 @@ extern "C" int nebo_transport_forward(const nebo_field_t* phiT, const nebo_field
   }
   if (!rc && cur != phiT->values)
     rc = check_hip(hipMemcpyAsync(phiT->values, cur, bytes, hipMemcpyDeviceToDevice, st), kCtx);
-  (void)hipFreeAsync(tmp, st);
+  scratch_free(tmp, st);
   return rc;
 }
 
