@@ -4,7 +4,11 @@
 // overlaps (k, then j, then i, as ParticleOperators.h:339-388 does) and sums
 // src(i,j,k) * fraction into a register.  ParticleToCell is a scatter whose
 // per-cell sums must come out in particle order to match the reference's serial
-// loop bit for bit (ParticleOperators.h:184-270), so atomics are out.  Instead:
+// loop bit for bit (ParticleOperators.h:184-270), so atomics on the cells are out.
+// The scatter by bricks (below, "ParticleToCell by bricks") gathers the particles of
+// one brick of cells in LDS and puts each cell's contributions in particle order
+// there.  Particle sets it does not suit (very many particles in one brick) are
+// sorted in device memory:
 //   1. count the cells each particle overlaps, exclusive scan -> entry offsets;
 //   2. each particle writes its entries in its own loop order: value
 //      src[p] * fraction and key cell at entry e, so entries stand in the serial
@@ -19,13 +23,16 @@
 // host when the index list is uploaded.
 
 #include "nebo_internal.h"
+#include "nebo_device.h"
 
 #include <hip/hip_runtime.h>
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <unordered_map>
 #include <vector>
 
@@ -224,6 +231,560 @@ __global__ void run_sum_kernel(double* __restrict__ dest, const uint32_t* __rest
   dest[cell] = acc;
 }
 
+// ---- ParticleToCell by bricks ------------------------------------------------------
+// The window is cut into bricks of 64 to 1024 cells.
+//   1. count_bricks: each block of a fixed share of the particles counts, in LDS, how
+//      many of them reach into each brick (one row of counts per block);
+//   2. scan_rows, scan_bricks: places of every block's records of every brick, by
+//      prefix sums over the rows of a brick and over the bricks;
+//   3. fill_bricks: the same blocks write a 48-byte record per particle and brick;
+//   4. sum_bricks: one workgroup per brick, a thread per cell: the records set their
+//      bits in the masks of the cells they reach, and each cell adds its contributions
+//      in the order of the bits (the serial loop's order).
+// Bound by the records' scattered writes (about 1.5 of them per particle of up to 1.5
+// cells) and by the arithmetic per contribution (75 % of sum_bricks' time issues
+// vector instructions), where a sort of the contributions moves 12 bytes of each (6.3
+// per particle) through memory 7 times.  2M particles of 0.2-1.5 cells on 112x96x104
+// cells: 342 us per call (sum_bricks 140, fill_bricks 118, count_bricks 25, the scans
+// 29) against 870 us sorted; 4M on 128^3: 575 against 1627; 1M on 40^3: 340 against
+// 711.
+
+struct Bricks {
+  int sh[3];     // log2 of a brick's cells per axis (at most 5)
+  int nb[3];     // bricks per axis
+  int total;     // bricks
+  bool has[3];   // axes the particles resolve
+};
+
+struct alignas(16) BrickRec {
+  double plo[3];
+  double size, src;
+  uint32_t idx;     // the particle
+  uint32_t range;   // first and last cell within the brick, 5 bits each, per axis
+};
+static_assert(sizeof(BrickRec) == 48, "record size");
+
+struct BrickStats {
+  uint64_t records;   // of all bricks
+  uint32_t most;      // of the fullest brick
+  uint32_t group;     // that one block writes into one brick, at most
+};
+
+constexpr int kBinThreads = 512;
+constexpr int kBinBatch = 4;          // particles a thread loads at a time
+constexpr int kBinRows = 512;          // blocks that bin the particles, at most
+constexpr int kRowCols = 16;           // bricks per block of scan_rows
+constexpr int kRowSegments = 64;
+constexpr int kMaxBricks = 16384;      // 64 KB of LDS counters
+constexpr int kBrickTarget = 512;      // particles per brick aimed at
+constexpr int kMostGroup = 32;         // records of one block in one brick
+// Particles per cell of the window: denser sets are sorted, since a cell's thread walks
+// its contributions alone (1M particles on 24^3 cells, 72 per cell: 1250 us by bricks,
+// 700 sorted; on 40^3, 16 per cell: 340 and 711).
+constexpr double kMostPerCell = 32;
+constexpr uint32_t kMostRecords = 1u << 17;   // records of one brick
+
+// Range of cells [lo, hi) of particle p, by particle_box's rules in 32-bit
+// arithmetic: values beyond 2^30 lie past any window either way.  False when the
+// particle is skipped; the range may be empty.
+struct PRange {
+  int lo[3], hi[3];
+  double plo[3];
+  double size;
+};
+
+struct PIn {
+  double c[3], size;
+};
+
+__device__ __forceinline__ PIn load_particle(const Coords& pc, const double* psize, long p)
+{
+  PIn v;
+  v.size = psize[p];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) v.c[a] = pc.c[a] ? pc.c[a][p] : 0;
+  return v;
+}
+
+__device__ __forceinline__ bool particle_range(const CellGrid& g, const Bricks& b, const PIn& v, PRange* r)
+{
+  r->size = v.size;
+  const double rp = v.size * 0.5;
+  bool ok = true;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    r->plo[a] = b.has[a] ? v.c[a] - rp : 0;
+    const double t = (r->plo[a] - g.loface[a]) / g.h[a];
+    if (!(t > -1.0)) ok = false;
+    r->lo[a] = (int)(t > 1.0e9 ? 1.0e9 : (t > 0.0 ? t : 0.0));
+    if (b.has[a]) {
+      const double phi = r->plo[a] + v.size;
+      double u = (phi - g.loface[a]) / g.h[a];
+      u = u > 1.0e9 ? 1.0e9 : (u < -2.0e9 ? -2.0e9 : u);
+      r->hi[a] = (int)u + 1;
+    } else {
+      r->hi[a] = r->lo[a] + 1;
+    }
+    if (r->hi[a] > g.nmax[a]) r->hi[a] = g.nmax[a];
+  }
+  return ok;
+}
+
+// f(brick, bx, by, bz) for every brick the range reaches into.
+template <typename F>
+__device__ __forceinline__ void for_bricks(const Bricks& b, const PRange& r, F&& f)
+{
+  if (r.hi[0] <= r.lo[0] || r.hi[1] <= r.lo[1] || r.hi[2] <= r.lo[2]) return;
+  for (int z = r.lo[2] >> b.sh[2]; z <= (r.hi[2] - 1) >> b.sh[2]; ++z)
+    for (int y = r.lo[1] >> b.sh[1]; y <= (r.hi[1] - 1) >> b.sh[1]; ++y)
+      for (int x = r.lo[0] >> b.sh[0]; x <= (r.hi[0] - 1) >> b.sh[0]; ++x)
+        f(x + b.nb[0] * (y + b.nb[1] * z), x, y, z);
+}
+
+__global__ __launch_bounds__(kBinThreads) void count_bricks(uint32_t* __restrict__ rows, CellGrid g, Bricks b,
+                                                            Coords pc, const double* __restrict__ psize, long np,
+                                                            int share, int* __restrict__ skipped)
+{
+  extern __shared__ uint32_t bins[];
+  for (int i = threadIdx.x; i < b.total; i += kBinThreads) bins[i] = 0;
+  __syncthreads();
+  const long first = (long)blockIdx.x * share, last = min(first + share, np);
+  for (long p0 = first + threadIdx.x; p0 < last; p0 += kBinBatch * kBinThreads) {
+    PIn in[kBinBatch];
+#pragma unroll
+    for (int u = 0; u < kBinBatch; ++u) in[u] = load_particle(pc, psize, min(p0 + u * kBinThreads, last - 1));
+#pragma unroll
+    for (int u = 0; u < kBinBatch; ++u) {
+      if (p0 + u * kBinThreads >= last) continue;
+      PRange r;
+      if (!particle_range(g, b, in[u], &r)) {
+        if (skipped) atomicAdd(skipped, 1);
+        continue;
+      }
+      for_bricks(b, r, [&](int brick, int, int, int) { atomicAdd(&bins[brick], 1u); });
+    }
+  }
+  __syncthreads();
+  uint32_t* row = rows + (size_t)blockIdx.x * b.total;
+  for (int i = threadIdx.x; i < b.total; i += kBinThreads) row[i] = bins[i];
+}
+
+// Each brick's counts become their exclusive prefix over the rows; totals[brick]
+// their sum, group[block] the largest count.  kRowCols bricks per block, the rows in
+// kRowSegments parts.
+__global__ __launch_bounds__(kRowCols * kRowSegments) void scan_rows(uint32_t* __restrict__ rows,
+                                                               uint32_t* __restrict__ totals,
+                                                               uint32_t* __restrict__ group, int n_rows,
+                                                               int n_bricks)
+{
+  constexpr int U = 8;   // loads in flight per thread
+  __shared__ uint32_t part[kRowSegments][kRowCols], bigs[kRowCols * kRowSegments / 64];
+  const int col = threadIdx.x % kRowCols, seg = threadIdx.x / kRowCols;
+  const int brick = blockIdx.x * kRowCols + col;
+  const int per = (n_rows + kRowSegments - 1) / kRowSegments;
+  const int r0 = min(seg * per, n_rows), r1 = min(r0 + per, n_rows);
+  uint32_t* mine = rows + min(brick, n_bricks - 1);
+  uint32_t sum = 0, big = 0, v[U] = {};
+  for (int r = r0; r < r1; r += U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = mine[(size_t)min(r + u, r1 - 1) * n_bricks];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (r + u < r1) sum += v[u];
+      big = max(big, v[u]);
+    }
+  }
+  part[seg][col] = sum;
+  big = brick < n_bricks ? big : 0;
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) big = max(big, (uint32_t)__shfl_xor((int)big, off, 64));
+  if ((threadIdx.x & 63) == 0) bigs[threadIdx.x >> 6] = big;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kRowCols * kRowSegments / 64; ++w) big = max(big, bigs[w]);
+    group[blockIdx.x] = big;
+  }
+  uint32_t at = 0;
+#pragma unroll
+  for (int q = 0; q < kRowSegments; ++q) at += q < seg ? part[q][col] : 0;
+  if (brick >= n_bricks) return;
+  for (int r = r0; r < r1; r += U) {
+    if (per > U) {   // else v holds the whole part
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = mine[(size_t)min(r + u, r1 - 1) * n_bricks];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (r + u < r1) mine[(size_t)(r + u) * n_bricks] = at;
+      at += v[u];
+    }
+  }
+  if (seg == kRowSegments - 1) totals[brick] = at;
+}
+
+// base[brick]: records before the brick's first (base[n_bricks]: all of them), and
+// the statistics the host chooses the next launch by.  One block, 1024 bricks at a
+// time.  (Where the records pass 2^32, base is not used.)
+__global__ __launch_bounds__(1024) void scan_bricks(uint32_t* __restrict__ base, const uint32_t* __restrict__ totals,
+                                                    int n_bricks, const uint32_t* __restrict__ group, int n_group,
+                                                    BrickStats* __restrict__ stats)
+{
+  __shared__ unsigned long long part[16];
+  __shared__ uint32_t bigs[16], groups[16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  unsigned long long before = 0;
+  uint32_t big = 0;
+  for (int i0 = 0; i0 < n_bricks; i0 += 1024) {
+    const int i = i0 + t;
+    const uint32_t own = i < n_bricks ? totals[i] : 0;
+    big = max(big, own);
+    unsigned long long sum = own;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const unsigned long long v = __shfl_up(sum, off, 64);
+      if (lane >= off) sum += v;
+    }
+    if (lane == 63) part[wave] = sum;
+    __syncthreads();
+    unsigned long long all = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      const unsigned long long v = part[w];
+      if (w < wave) sum += v;
+      all += v;
+    }
+    if (i < n_bricks) base[i] = (uint32_t)(before + sum - own);
+    before += all;
+    __syncthreads();
+  }
+  uint32_t grp = 0;
+  for (int i = t; i < n_group; i += 1024) grp = max(grp, group[i]);
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    big = max(big, (uint32_t)__shfl_xor((int)big, off, 64));
+    grp = max(grp, (uint32_t)__shfl_xor((int)grp, off, 64));
+  }
+  if (lane == 0) {
+    bigs[wave] = big;
+    groups[wave] = grp;
+  }
+  __syncthreads();
+  if (t == 0) {
+    for (int w = 1; w < 16; ++w) {
+      big = max(big, bigs[w]);
+      grp = max(grp, groups[w]);
+    }
+    base[n_bricks] = (uint32_t)before;
+    stats->records = before;
+    stats->most = big;
+    stats->group = grp;
+  }
+}
+
+__global__ __launch_bounds__(kBinThreads) void fill_bricks(BrickRec* __restrict__ recs,
+                                                           const uint32_t* __restrict__ rows,
+                                                           const uint32_t* __restrict__ base, CellGrid g, Bricks b,
+                                                           Coords pc, const double* __restrict__ psize,
+                                                           const double* __restrict__ src, long np, int share)
+{
+  extern __shared__ uint32_t bins[];
+  const uint32_t* row = rows + (size_t)blockIdx.x * b.total;
+  for (int i = threadIdx.x; i < b.total; i += kBinThreads) bins[i] = base[i] + row[i];
+  __syncthreads();
+  const long first = (long)blockIdx.x * share, last = min(first + share, np);
+  for (long p0 = first + threadIdx.x; p0 < last; p0 += kBinBatch * kBinThreads) {
+    PIn in[kBinBatch];
+    double val[kBinBatch];
+#pragma unroll
+    for (int u = 0; u < kBinBatch; ++u) {
+      const long p = min(p0 + u * kBinThreads, last - 1);
+      in[u] = load_particle(pc, psize, p);
+      val[u] = src[p];
+    }
+#pragma unroll
+    for (int u = 0; u < kBinBatch; ++u) {
+      const long p = p0 + u * kBinThreads;
+      PRange r;
+      if (p >= last || !particle_range(g, b, in[u], &r)) continue;
+      BrickRec rec;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) rec.plo[a] = r.plo[a];
+      rec.size = r.size;
+      rec.src = val[u];
+      rec.idx = (uint32_t)p;
+      for_bricks(b, r, [&](int brick, int x, int y, int z) {
+        const int at[3] = {x, y, z};
+        rec.range = 0;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          const int o = at[a] << b.sh[a], m = (1 << b.sh[a]) - 1;
+          const int lo = max(r.lo[a] - o, 0), hi = min(r.hi[a] - 1 - o, m);
+          rec.range |= (uint32_t)(lo | hi << 5) << (10 * a);
+        }
+        recs[atomicAdd(&bins[brick], 1u)] = rec;
+      });
+    }
+  }
+}
+
+// f(cell) for the cells of a record's range, x fastest.
+template <typename F>
+__device__ __forceinline__ void for_range(const Bricks& b, uint32_t range, F&& f)
+{
+  const int x0 = range & 31, x1 = (range >> 5) & 31, y0 = (range >> 10) & 31, y1 = (range >> 15) & 31;
+  const int z0 = (range >> 20) & 31, z1 = (range >> 25) & 31;
+  for (int z = z0; z <= z1; ++z)
+    for (int y = y0; y <= y1; ++y)
+      for (int x = x0; x <= x1; ++x) f(x | (y | z << b.sh[1]) << b.sh[0]);
+}
+
+__device__ __forceinline__ double cube_volume(const Bricks& b, double size)
+{
+  const double rp = size * 0.5;
+  return (b.has[0] ? 2 * rp : 1) * (b.has[1] ? 2 * rp : 1) * (b.has[2] ? 2 * rp : 1);
+}
+
+// One workgroup per brick, NT threads with Q cells each.  The brick's records are
+// taken R at a time in the order of their particles.  A record goes to LDS, where it
+// also sets its bit in the mask of every cell it reaches; each cell's thread then
+// walks its mask's bits upwards, which is particle order, and adds the contributions
+// it forms from the records.
+//
+// The blocks that wrote the records hold consecutive particles, so a brick's list is
+// in order up to the records one block wrote (at most `group` of them, 1.4 on average
+// in the case above): a record's place follows from its neighbours.  `share` is the
+// particles per block.
+template <int NT, int Q, int R>
+__global__ __launch_bounds__(NT) void sum_bricks(double* __restrict__ dest, CellGrid g, Bricks b,
+                                                 const uint32_t* __restrict__ base,
+                                                 const BrickRec* __restrict__ recs, uint32_t share, int group)
+{
+  constexpr int C = NT * Q;      // cells, at most
+  constexpr int W = R / 64;      // mask words per cell
+  __shared__ double plo[3][R], size[R], val[R];
+  __shared__ unsigned long long mask[W][C];
+  __shared__ uint32_t idx[R + 4 * (kMostGroup - 1)];
+
+  const int brick = xcd_tile(blockIdx.x, gridDim.x);
+  const uint32_t first = base[brick];
+  const int n = (int)(base[brick + 1] - first);
+  if (n == 0) return;
+  const BrickRec* mine = recs + first;
+  const int t = threadIdx.x;
+  const int cells = 1 << (b.sh[0] + b.sh[1] + b.sh[2]);
+  const int ox = (brick % b.nb[0]) << b.sh[0];
+  const int oy = (brick / b.nb[0] % b.nb[1]) << b.sh[1];
+  const int oz = (brick / b.nb[0] / b.nb[1]) << b.sh[2];
+  const int M = group - 1;       // a record is at most M places from its own
+
+  double acc[Q], lo[Q][3], hi[Q][3];
+  long at[Q];   // flat index of the cell, -1 outside the window
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int c = t + q * NT;
+    const int x = ox + (c & ((1 << b.sh[0]) - 1)), y = oy + ((c >> b.sh[0]) & ((1 << b.sh[1]) - 1));
+    const int z = oz + (c >> (b.sh[0] + b.sh[1]));
+    const int xyz[3] = {x, y, z};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      lo[q][a] = g.loface[a] + (double)xyz[a] * g.h[a];
+      hi[q][a] = lo[q][a] + g.h[a];
+    }
+    at[q] = -1;
+    acc[q] = 0.0;
+    if (c < cells && x < g.nmax[0] && y < g.nmax[1] && z < g.nmax[2]) {
+      const long gx = g.glob[0] > 1 ? x + g.off[0] : 0, gy = g.glob[1] > 1 ? y + g.off[1] : 0;
+      const long gz = g.glob[2] > 1 ? z + g.off[2] : 0;
+      at[q] = gx + (long)g.glob[0] * (gy + (long)g.glob[1] * gz);
+      acc[q] = dest[at[q]];
+    }
+  }
+
+  for (int r0 = 0; r0 < n; r0 += R) {
+    // the particles of places r0 - 2M .. r0 + R + 2M, and empty masks
+    for (int i = t; i < R + 4 * M; i += NT) {
+      const int j = r0 - 2 * M + i;
+      idx[i] = j >= 0 && j < n ? mine[j].idx : 0xffffffffu;   // no particle's block
+    }
+    for (int i = t; i < W * C; i += NT) mask[i / C][i % C] = 0;
+    __syncthreads();
+    for (int i = M + t; i < R + 3 * M; i += NT) {
+      const int j = r0 - 2 * M + i;
+      if (j < 0 || j >= n) continue;
+      const uint32_t p = idx[i], blk = p / share;
+      int place = j - r0;
+      for (int k = i - 1; k >= i - M && idx[k] / share == blk; --k) place -= idx[k] > p;
+      for (int k = i + 1; k <= i + M && idx[k] / share == blk; ++k) place += idx[k] < p;
+      if (place < 0 || place >= R) continue;
+      const BrickRec r = mine[j];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) plo[a][place] = r.plo[a];
+      size[place] = r.size;
+      val[place] = r.src;
+      unsigned long long* word = mask[place >> 6];
+      for_range(b, r.range, [&](int c) { atomicOr(&word[c], 1ull << (place & 63)); });
+    }
+    __syncthreads();
+    const int words = min(W, (n - r0 + 63) / 64);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int c = t + q * NT;
+      int w = 0;
+      unsigned long long m = mask[0][c];
+      for (;;) {
+        while (m == 0 && ++w < words) m = mask[w][c];
+        if (w >= words) break;
+        const int i = w * 64 + __builtin_ctzll(m);
+        m &= m - 1;
+        const double s = size[i];
+        double part[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          const double pl = plo[a][i], ph = pl + s;
+          part[a] = b.has[a] ? __builtin_fmin(hi[q][a], ph) - __builtin_fmax(lo[q][a], pl) : 1;
+        }
+        acc[q] += val[i] * (part[0] * part[1] * part[2] / cube_volume(b, s));
+      }
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+    if (at[q] >= 0) dest[at[q]] = acc[q];
+}
+
+using SumBricksFn = void (*)(double*, CellGrid, Bricks, const uint32_t*, const BrickRec*, uint32_t, int);
+SumBricksFn sum_bricks_fn(int cells, int* threads)
+{
+  *threads = cells <= 64 ? 64 : cells <= 128 ? 128 : 256;
+  return cells <= 64    ? sum_bricks<64, 1, 128>
+         : cells <= 128 ? sum_bricks<128, 1, 128>
+         : cells <= 256 ? sum_bricks<256, 1, 256>
+         : cells <= 512 ? sum_bricks<256, 2, 256>
+                        : sum_bricks<256, 4, 128>;
+}
+
+// Brick shape for np particles on the window: about kBrickTarget particles per
+// brick, within 64 to 1024 cells (fewer on windows of fewer resolved axes) and
+// kMaxBricks bricks.  False where that many bricks do not cover the window.
+bool choose_bricks(const CellGrid& g, const Coords& pc, int64_t np, Bricks* b)
+{
+  const double window = (double)g.nmax[0] * g.nmax[1] * g.nmax[2];
+  if (np > kMostPerCell * window) return false;
+  int bits = 6;
+  while (bits < 10 && np / window * (double)(2 << bits) <= kBrickTarget) ++bits;
+  for (;; ++bits) {
+    int used = 0;
+    for (int a = 0; a < 3; ++a) b->sh[a] = 0;
+    for (; used < bits; ++used) {
+      int pick = -1;
+      for (int a = 0; a < 3; ++a)
+        if (b->sh[a] < 5 && (1 << b->sh[a]) < g.nmax[a] && (pick < 0 || b->sh[a] < b->sh[pick])) pick = a;
+      if (pick < 0) break;
+      ++b->sh[pick];
+    }
+    double total = 1;
+    for (int a = 0; a < 3; ++a) {
+      b->nb[a] = (g.nmax[a] + (1 << b->sh[a]) - 1) >> b->sh[a];
+      b->has[a] = pc.c[a] != nullptr;
+      total *= b->nb[a];
+    }
+    if (total <= kMaxBricks) {
+      b->total = (int)total;
+      return true;
+    }
+    if (bits >= 10 || used < bits) return false;
+  }
+}
+
+// Page-locked slots the statistics are written to, one per call in progress.
+std::mutex g_stats_mu;
+std::vector<BrickStats*> g_stats_free;
+
+int take_stats(BrickStats** s, const char* ctx)
+{
+  std::lock_guard<std::mutex> lk(g_stats_mu);
+  if (!g_stats_free.empty()) {
+    *s = g_stats_free.back();
+    g_stats_free.pop_back();
+    return NEBO_OK;
+  }
+  return check_hip(hipHostMalloc((void**)s, sizeof(BrickStats), hipHostMallocPortable | hipHostMallocMapped), ctx);
+}
+
+void give_stats(BrickStats* s)
+{
+  std::lock_guard<std::mutex> lk(g_stats_mu);
+  g_stats_free.push_back(s);
+}
+
+// The scatter by bricks.  *counted: the particles were counted (and the skipped ones
+// reported); *done: dest holds the sums.  Left to the sort when *done stays false:
+// windows of too many bricks, and sets crowded into few bricks (more than
+// kMostRecords records in one, whose workgroup would walk them alone, or more than
+// kMostGroup of one block in one, which are ordered by comparing neighbours).
+int scatter_by_bricks(double* dest, const double* src, const CellGrid& g, const Coords& pc, const double* psize,
+                      int64_t np, int32_t* skipped, hipStream_t s, const char* ctx, bool* counted, bool* done)
+{
+  *counted = *done = false;
+  Bricks b;
+  if (np >= (int64_t(1) << 31) || !choose_bricks(g, pc, np, &b)) return NEBO_OK;
+  // at most kBinRows rows, more where the bricks are few (dense sets), so that one
+  // block's records of one brick stay few
+  const int64_t most_rows = std::max<int64_t>(kBinRows, (int64_t)kBinRows * 4096 / b.total);
+  const int n_rows = (int)std::min<int64_t>(most_rows, (np + 1023) / 1024);
+  const int share = (int)((np + n_rows - 1) / n_rows);
+  const size_t row_bytes = sizeof(uint32_t) * (size_t)b.total;
+  char* work = nullptr;
+  BrickStats* stats = nullptr;
+  int rc = take_stats(&stats, ctx);
+  if (rc) return rc;
+  // rows, totals, base (+1), group (one per block of scan_rows)
+  const int n_group = (b.total + kRowCols - 1) / kRowCols;
+  if ((rc = scratch_alloc((void**)&work, row_bytes * (n_rows + 2) + sizeof(uint32_t) * (1 + n_group), s, ctx))) {
+    give_stats(stats);
+    return rc;
+  }
+  uint32_t* rows = reinterpret_cast<uint32_t*>(work);
+  uint32_t* totals = rows + (size_t)n_rows * b.total;
+  uint32_t* base = totals + b.total;
+  uint32_t* group = base + b.total + 1;
+  hipLaunchKernelGGL(count_bricks, dim3(n_rows), dim3(kBinThreads), row_bytes, s, rows, g, b, pc, psize, (long)np,
+                     share, skipped);
+  hipLaunchKernelGGL(scan_rows, dim3(n_group), dim3(kRowCols * kRowSegments), 0, s,
+                     rows, totals, group, n_rows,
+                     b.total);
+  hipLaunchKernelGGL(scan_bricks, dim3(1), dim3(1024), 0, s, base, totals, b.total, group, n_group,
+                     stats);
+  rc = check_hip(hipGetLastError(), ctx);
+  if (!rc) rc = check_hip(hipStreamSynchronize(s), ctx);
+  const BrickStats st = *stats;
+  give_stats(stats);
+  if (rc) {
+    scratch_free(work, s);
+    return rc;
+  }
+  *counted = true;
+  if (st.records > 0 && st.most <= kMostRecords && st.group <= kMostGroup && st.records < (uint64_t(1) << 31)) {
+    BrickRec* recs = nullptr;
+    if (!(rc = scratch_alloc((void**)&recs, sizeof(BrickRec) * st.records, s, ctx))) {
+      hipLaunchKernelGGL(fill_bricks, dim3(n_rows), dim3(kBinThreads), row_bytes, s, recs, rows, base, g, b, pc,
+                         psize, src, (long)np, share);
+      int threads = 0;
+      const SumBricksFn fn = sum_bricks_fn(1 << (b.sh[0] + b.sh[1] + b.sh[2]), &threads);
+      hipLaunchKernelGGL(fn, dim3(b.total), dim3(threads), 0, s, dest, g, b, base, recs, (uint32_t)share,
+                         (int)st.group);
+      rc = check_hip(hipGetLastError(), ctx);
+      scratch_free(recs, s);
+    }
+    *done = rc == NEBO_OK;
+  } else if (st.records == 0) {
+    *done = true;
+  }
+  scratch_free(work, s);
+  return rc;
+}
+
 int bits_for(uint64_t n)   // bits to hold 0..n-1
 {
   int b = 0;
@@ -301,6 +862,12 @@ extern "C" int nebo_particle_to_cell(const nebo_field_t* dest, const double* src
   hipStream_t s = (hipStream_t)stream;
   const CellGrid g = make_grid(dest, *geom);
   const Coords pc{{px, py, pz}};
+  {
+    bool counted = false, done = false;
+    rc = scatter_by_bricks(static_cast<double*>(dest->values), src, g, pc, psize, np, skipped, s, ctx, &counted, &done);
+    if (rc || done) return rc;
+    if (counted) skipped = nullptr;
+  }
   const unsigned blocks = (unsigned)((np + kBlock - 1) / kBlock);
   long* counts = nullptr;
   long* offsets = nullptr;
