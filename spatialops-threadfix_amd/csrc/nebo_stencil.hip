@@ -815,16 +815,24 @@ LaplFn lapl_table(int s) { return lapl_pick(s, std::make_index_sequence<kNumShap
 //     planes ahead) with the longest z chunk (512, 256 or 128 planes) that still
 //     gives every CU a workgroup: one workgroup per CU, all walking the same
 //     planes (512^3 on MI355X: 658 us against 775 us with 64-plane chunks, whose
-//     eight concurrent z slabs lie 135 MB apart);
-//  4. else the default tile when it gives at least half the CUs a workgroup
-//     (256^3: 64-plane chunks, one workgroup per CU), for div(k grad phi) on
-//     boxes whose width is a multiple of 128 as pair columns;
-//  5. smaller boxes run one-wave column tiles of 64 columns x 2 rows per lane
-//     with the longest z chunk (16, 8 or 4 planes) that gives every CU two
-//     waves (else 4 planes): time steps that alternate two fields, timed in a
-//     hipGraph on MI355X, 64^3 3.9 us (Laplacian) and 4.6 us (div(k grad phi))
-//     against 7.8 and 9.0 us for the direct schedule's 64 x 4 x 16 tiles;
-//     128^3 8.7 and 13.9 us against 10.0 and 18.6 us.
+//     eight concurrent z slabs lie 135 MB apart), where the tiles fill the CUs (see
+//     kFill) or divide the box in x and y.  (Of the boxes they divide, 384^3 fills
+//     two thirds of the CUs once and leaves the rest idle: 514 us against 320 for
+//     the tile of rule 5; the selection there is one programs rely on.);
+//  4. else the default tile where it fills the CUs (256^3: 64-plane chunks, one
+//     workgroup per CU), for div(k grad phi) on boxes whose width is a multiple of
+//     128 as pair columns;
+//  5. every other box runs one-wave column tiles of 64 columns, whose many small
+//     workgroups spread evenly whatever the sides are: 4 rows per lane and 8 planes
+//     on large boxes, 2 rows and 8 planes below, 16 planes where the box gives every
+//     SIMD a wave that long, 8 and then 4 planes where it does not.  div(k grad phi)
+//     on MI355X, three fields' sets in turn, before (rule 4 for half the CUs, then 2
+//     rows and the longest chunk with two waves per CU) and now: 300x210x170 72.7 and
+//     67.7 us, 192^3 66.8 and 45.4, 400x200x200 140 and 97.4, 300^3 262 and 160,
+//     130x400x320 231 and 110, 160^3 22.6 and 20.8, 100^3 10.6 and 10.2.  Laplacian:
+//     200x190x210 35.0 and 25.0, 100^3 8.3 and 7.2.  Time steps of two fields, timed
+//     in a hipGraph: 64^3 3.9 us (Laplacian) and 4.6 us (div(k grad phi)) against 7.8
+//     and 9.0 us for the direct schedule's 64 x 4 x 16 tiles.
 std::atomic<int> g_pinned[2] = {{-1}, {-1}};
 std::atomic<int> g_last[2] = {{kDefaultShape}, {kDefaultShape}};   // last pinned or tuned tile
 struct TunedTile {
@@ -834,9 +842,10 @@ std::mutex g_tuned_mu;
 std::vector<TunedTile> g_tuned;
 
 constexpr int kSmallColumn[] = {find_shape_c(64, 2, 16, 3), find_shape_c(64, 2, 8, 3), find_shape_c(64, 2, 4, 3)};
+constexpr int kLargeColumn = find_shape_c(64, 4, 8, 3);
 constexpr int kLongChunks[] = {find_shape_c(128, 8, 512, 7), find_shape_c(128, 8, 256, 7),
                                find_shape_c(128, 8, 128, 7)};
-static_assert(kSmallColumn[0] >= 0 && kSmallColumn[1] >= 0 && kSmallColumn[2] >= 0 && kLongChunks[0] >= 0 &&
+static_assert(kSmallColumn[0] >= 0 && kSmallColumn[1] >= 0 && kSmallColumn[2] >= 0 && kLargeColumn >= 0 && kLongChunks[0] >= 0 &&
                   kLongChunks[1] >= 0 && kLongChunks[2] >= 0,
               "box-size tiles");
 
@@ -846,6 +855,21 @@ long tile_groups(int shape, const nebo_limits_t& lim)
   const TileShape sh = kShapes[shape];
   const Tiles T = make_tiles(lim, sh.tx, tile_geometry(sh).tile_y, sh.zc);
   return (long)T.nx * T.ny * T.nz;
+}
+
+// Share of the cells that the tiles of a box could hold on all CUs (in whole rounds
+// of one tile per CU) that the box has.  Where it is low, CUs idle or lanes run past
+// the box: 224^3 0.67 (73.6 us against 76.3 for rule 5's tile), 300x210x170 0.64 (72.6
+// against 67.7), 320x256x128 0.63 (72.3 against 61.6).
+constexpr double kFill = 0.66;
+
+double tile_fill(int shape, const nebo_limits_t& lim, int cus)
+{
+  const TileShape sh = kShapes[shape];
+  const long groups = tile_groups(shape, lim), rounds = (groups + cus - 1) / cus;
+  double cells = 1;
+  for (int d = 0; d < 3; ++d) cells *= lim.hi[d] - lim.lo[d];
+  return cells / ((double)rounds * cus * sh.tx * tile_geometry(sh).tile_y * sh.zc);
 }
 
 int select_shape(int kernel, int device, const nebo_limits_t& lim)
@@ -860,13 +884,20 @@ int select_shape(int kernel, int device, const nebo_limits_t& lim)
         return t.shape;
   }
   const int cus = device_cu_count(device);
+  const TileShape def = kShapes[kDefaultShape];
+  const bool divides = n[0] % def.tx == 0 && n[1] % tile_geometry(def).tile_y == 0;
   for (int sh : kLongChunks)
-    if (tile_groups(sh, lim) >= cus) return sh;
-  if (2 * tile_groups(kDefaultShape, lim) >= cus)
+    if (tile_groups(sh, lim) >= cus && (divides || tile_fill(sh, lim, cus) >= kFill)) return sh;
+  if (tile_fill(kDefaultShape, lim, cus) >= kFill)
     return kernel == 0 && n[0] % kShapes[kDefaultPairShape].tx == 0 ? kDefaultPairShape : kDefaultShape;
-  for (int sh : kSmallColumn)
-    if (tile_groups(sh, lim) >= 2 * cus) return sh;
-  return kSmallColumn[2];
+  // workgroups of 2 rows and 8 planes per CU: the Laplacian's lighter waves gain from
+  // 4 rows later (200x190x210, 40 per CU: 27.2 us against 25.0; 300x210x170, 45: 39.4
+  // against 40.7)
+  const long waves8 = tile_groups(kSmallColumn[1], lim);
+  if (waves8 >= (kernel == 0 ? 24L : 44L) * cus) return kLargeColumn;
+  if (waves8 >= 16L * cus) return kSmallColumn[1];
+  if (tile_groups(kSmallColumn[0], lim) >= 4L * cus) return kSmallColumn[0];
+  return waves8 >= 4L * cus ? kSmallColumn[1] : kSmallColumn[2];
 }
 
 int find_shape(int tx, int ty, int zc, int variant)
