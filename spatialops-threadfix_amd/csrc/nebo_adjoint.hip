@@ -64,8 +64,6 @@ size_t field_npts(const nebo_field_t* f) { return (size_t)f->glob[0] * f->glob[1
 namespace {
 
 constexpr int kTx = 64;
-constexpr int kTy = 4;
-constexpr int kZChunk = 16;
 
 struct FaceQ {
   double kw;  // kf * w
@@ -83,7 +81,7 @@ __device__ __forceinline__ FaceQ face_q(double lam_lo, double lam_hi, double p_l
   return FaceQ{kf * w, w * gp};
 }
 
-__global__ __launch_bounds__(kTx * kTy) void adjoint_kernel(
+__global__ __launch_bounds__(1024) void adjoint_kernel(
     double* __restrict__ lam_out, double* __restrict__ gk, const double* __restrict__ lam,
     const double* __restrict__ p, const double* __restrict__ k, Box3 B, int X, int XY,
     nebo_axis_coefs_t c, double dt)
@@ -94,10 +92,12 @@ __global__ __launch_bounds__(kTx * kTy) void adjoint_kernel(
   const int ty = rest % B.ny;
   const int tz = rest / B.ny;
   const int x = tx * kTx + (threadIdx.x & (kTx - 1));
-  const int y = ty * kTy + (threadIdx.x / kTx);
+  const int wave = threadIdx.x / kTx;
+  const int y = ty * B.rows + wave % B.rows;
   if (x >= B.n[0] || y >= B.n[1]) return;
-  const int z0 = tz * B.zc;
-  const int z1 = min(z0 + B.zc, B.n[2]);
+  const int z0 = tz * B.zc + wave / B.rows * B.wz;
+  const int z1 = min(min(z0 + B.wz, (tz + 1) * B.zc), B.n[2]);
+  if (z0 >= z1) return;
   const double i0x = c.interp[0][0], i1x = c.interp[0][1], g0x = c.grad[0][0], g1x = c.grad[0][1];
   const double i0y = c.interp[1][0], i1y = c.interp[1][1], g0y = c.grad[1][0], g1y = c.grad[1][1];
   const double i0z = c.interp[2][0], i1z = c.interp[2][1], g0z = c.grad[2][0], g1z = c.grad[2][1];
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(kTx * kTy) void adjoint_kernel(
   double lc = lam[i], pc = p[i], kc = k[i];
   FaceQ zlo = face_q(lam[i - XY], lc, p[i - XY], pc, k[i - XY], kc, d0z, d1z, g0z, g1z, i0z, i1z);
   for (int z = z0; z < z1; ++z, i += XY) {
-    const double lz = lam[i + XY], pz = p[i + XY], kz = k[i + XY];
+    const double lz = lam[i + XY], pz = p[i + XY], kz = k[i + XY], gc = gk[i];
     const FaceQ xlo = face_q(lam[i - 1], lc, p[i - 1], pc, k[i - 1], kc, d0x, d1x, g0x, g1x, i0x, i1x);
     const FaceQ xhi = face_q(lc, lam[i + 1], pc, p[i + 1], kc, k[i + 1], d0x, d1x, g0x, g1x, i0x, i1x);
     const FaceQ ylo = face_q(lam[i - X], lc, p[i - X], pc, k[i - X], kc, d0y, d1y, g0y, g1y, i0y, i1y);
@@ -120,13 +120,131 @@ __global__ __launch_bounds__(kTx * kTy) void adjoint_kernel(
     const double bx = xhi.wg * i0x + xlo.wg * i1x;
     const double by = yhi.wg * i0y + ylo.wg * i1y;
     const double bz = zhi.wg * i0z + zlo.wg * i1z;
-    lam_out[i] = lc + dt * ((ax + ay) + az);
-    gk[i] = gk[i] + dt * ((bx + by) + bz);
+    const double v = lc + dt * ((ax + ay) + az);
+    lam_out[i] = v;
+    store_images(&lam_out[i], x, y, z, B.n, X, XY, v);
+    gk[i] = gc + dt * ((bx + by) + bz);
     lc = lz;
     pc = pz;
     kc = kz;
     zlo = zhi;
   }
+}
+
+// Column schedule (the layout of the stencil kernels' one-wave column tiles): a wave
+// of 64 x columns, each lane RY rows of its column marching zc planes; lam, phi and k
+// on the rows plus one halo row each side in PF + 1 rotated register slots (loads PF
+// planes ahead), g_k on the lane's rows, x neighbours from the adjacent lanes (DPP)
+// and at the wave's ends from the edge loads (readlane).  Every cell is evaluated in
+// adjoint_kernel's order, so the two are bit-identical.
+template <int RY, int PF, int SP>
+__global__ __launch_bounds__(kLanes) void adjoint_column_kernel(
+    double* __restrict__ lam_out, double* __restrict__ gk, const double* __restrict__ lam,
+    const double* __restrict__ p, const double* __restrict__ k, Tiles T, int zc, int X, int XY,
+    nebo_axis_coefs_t c, double dt)
+{
+  const int t = xcd_tile(blockIdx.x, gridDim.x);
+  const int tx = t % T.nx;
+  const int rest = t / T.nx;
+  const int ty = rest % T.ny;
+  const int tz = rest / T.ny;
+  const int lane = threadIdx.x;
+  const int xw0 = T.lo[0] + tx * kLanes, x = xw0 + lane;
+  const int y0 = T.lo[1] + ty * RY;
+  const int z0 = T.lo[2] + tz * zc;
+  const int z1 = min(z0 + zc, T.hi[2]);
+  const bool xin = x < T.hi[0];
+  const ColumnGeom<RY> g = column_geom<RY>(T, X, xw0, y0, lane);
+  const double i0x = c.interp[0][0], i1x = c.interp[0][1], g0x = c.grad[0][0], g1x = c.grad[0][1];
+  const double i0y = c.interp[1][0], i1y = c.interp[1][1], g0y = c.grad[1][0], g1y = c.grad[1][1];
+  const double i0z = c.interp[2][0], i1z = c.interp[2][1], g0z = c.grad[2][0], g1z = c.grad[2][1];
+  const double d0x = c.div[0][0], d1x = c.div[0][1], d0y = c.div[1][0], d1y = c.div[1][1];
+  const double d0z = c.div[2][0], d1z = c.div[2][1];
+
+  struct Col { double l[RY + 2], p[RY + 2], k[RY + 2], le, pe, ke, gk[RY]; };
+  auto load = [&](int z) __attribute__((always_inline)) {
+    Col v;
+    const Rsrc lb = plane_rsrc(plane_base(lam, T, X, XY, z), X, XY);
+    const Rsrc pb = plane_rsrc(plane_base(p, T, X, XY, z), X, XY);
+    const Rsrc kb = plane_rsrc(plane_base(k, T, X, XY, z), X, XY);
+    const Rsrc gb = plane_rsrc(plane_base(static_cast<const double*>(gk), T, X, XY, z), X, XY);
+#pragma unroll
+    for (int q = 0; q < RY + 2; ++q) {
+      v.l[q] = load_at(lb, g.row[q]);
+      v.p[q] = load_at(pb, g.row[q]);
+      v.k[q] = load_at(kb, g.row[q]);
+    }
+    v.le = load_at(lb, g.edge);
+    v.pe = load_at(pb, g.edge);
+    v.ke = load_at(kb, g.edge);
+#pragma unroll
+    for (int j = 0; j < RY; ++j) v.gk[j] = load_at(gb, g.row[j + 1]);
+    return v;
+  };
+  constexpr int NS = PF + 1;
+  Col S[NS];
+#pragma unroll
+  for (int q = 0; q < NS; ++q) S[q] = load(min(z0 + q, z1));
+  FaceQ zlo[RY];
+  {
+    const Rsrc lb = plane_rsrc(plane_base(lam, T, X, XY, z0 - 1), X, XY);
+    const Rsrc pb = plane_rsrc(plane_base(p, T, X, XY, z0 - 1), X, XY);
+    const Rsrc kb = plane_rsrc(plane_base(k, T, X, XY, z0 - 1), X, XY);
+#pragma unroll
+    for (int j = 0; j < RY; ++j)
+      zlo[j] = face_q(load_at(lb, g.row[j + 1]), S[0].l[j + 1], load_at(pb, g.row[j + 1]), S[0].p[j + 1],
+                      load_at(kb, g.row[j + 1]), S[0].k[j + 1], d0z, d1z, g0z, g1z, i0z, i1z);
+  }
+  auto step = [&](auto JJ, const int z) __attribute__((always_inline)) {
+    constexpr int jj = decltype(JJ)::value;
+    const Col& C0 = S[jj];
+    const Col& C1 = S[(jj + 1) % NS];
+    const Rsrc ob = plane_rsrc(plane_base(lam_out, T, X, XY, z), X, XY);
+    const Rsrc gb = plane_rsrc(plane_base(gk, T, X, XY, z), X, XY);
+    // the y face between rows j-1 and j is formed once, as row j-1's high face
+    FaceQ ylo = face_q(C0.l[0], C0.l[1], C0.p[0], C0.p[1], C0.k[0], C0.k[1], d0y, d1y, g0y, g1y, i0y, i1y);
+#pragma unroll
+    for (int j = 0; j < RY; ++j) {
+      const double lc = C0.l[j + 1], pc = C0.p[j + 1], kc = C0.k[j + 1];
+      const double ll = from_lower_lane(lc), lu = from_upper_lane(lc);
+      const double pl = from_lower_lane(pc), pu = from_upper_lane(pc);
+      const double kl = from_lower_lane(kc), ku = from_upper_lane(kc);
+      // lane reads outside the selects: every lane takes them (see lane_value)
+      const double lel = lane_value(C0.le, j), ler = lane_value(C0.le, 32 + j);
+      const double pel = lane_value(C0.pe, j), per = lane_value(C0.pe, 32 + j);
+      const double kel = lane_value(C0.ke, j), ker = lane_value(C0.ke, 32 + j);
+      const bool first = lane == 0, last = lane == kLanes - 1;
+      const FaceQ xlo = face_q(first ? lel : ll, lc, first ? pel : pl, pc, first ? kel : kl, kc, d0x, d1x, g0x, g1x,
+                               i0x, i1x);
+      const FaceQ xhi = face_q(lc, last ? ler : lu, pc, last ? per : pu, kc, last ? ker : ku, d0x, d1x, g0x, g1x,
+                               i0x, i1x);
+      const FaceQ yhi = face_q(lc, C0.l[j + 2], pc, C0.p[j + 2], kc, C0.k[j + 2], d0y, d1y, g0y, g1y, i0y, i1y);
+      const FaceQ zhi = face_q(lc, C1.l[j + 1], pc, C1.p[j + 1], kc, C1.k[j + 1], d0z, d1z, g0z, g1z, i0z, i1z);
+      const double ax = xhi.kw * g0x + xlo.kw * g1x;
+      const double ay = yhi.kw * g0y + ylo.kw * g1y;
+      const double az = zhi.kw * g0z + zlo[j].kw * g1z;
+      const double bx = xhi.wg * i0x + xlo.wg * i1x;
+      const double by = yhi.wg * i0y + ylo.wg * i1y;
+      const double bz = zhi.wg * i0z + zlo[j].wg * i1z;
+      const double v = lc + dt * ((ax + ay) + az);
+      const double gnew = C0.gk[j] + dt * ((bx + by) + bz);
+      ylo = yhi;
+      zlo[j] = zhi;
+      if (xin && y0 + j < T.hi[1]) {
+        store_at<SP>(ob, g.row[j + 1], v);
+        store_at<SP>(gb, g.row[j + 1], gnew);
+        store_column_images<SP>(lam_out, T, X, XY, z, g.row[j + 1], image_step(x, T.hi[0], 8),
+                                image_step(y0 + j, T.hi[1], 8 * X), v);
+      }
+    }
+    S[jj] = load(min(z + NS, z1));
+  };
+  const int full = (z1 - z0) / NS, rem = (z1 - z0) - NS * full;
+  int z = z0;
+  for (int q = 0; q < full; ++q, z += NS)
+    unroll_steps([&](auto J) { step(J, z + decltype(J)::value); }, std::make_integer_sequence<int, NS>{});
+  unroll_steps([&](auto J) { if (rem > decltype(J)::value) step(J, z + decltype(J)::value); },
+               std::make_integer_sequence<int, NS - 1>{});
 }
 
 const char* kCtx = "Nebo Adjoint";
@@ -136,36 +254,49 @@ int check_periodic_field(const nebo_field_t* f, const nebo_field_t* ref)
   return check_periodic_operand(f, ref, kCtx);
 }
 
-// out = phi + dt*div(interp(k)*grad(phi)), then out's periodic ghosts.  phi's
-// ghosts must already hold the periodic images.
+// out = phi + dt*div(interp(k)*grad(phi)) and out's periodic ghosts (the kernel writes
+// both).  phi's ghosts must already hold the periodic images.
 int step_filled(const nebo_field_t* out, const nebo_field_t* phi, const nebo_field_t* k,
                 const nebo_axis_coefs_t& c, double dt, void* stream)
 {
-  int rc = launch_diffusion_euler(out, k, phi, c, dt, interior_of(out), stream);
-  if (rc) return rc;
-  return fill_ghosts_periodic(out, stream);
+  return launch_diffusion_euler(out, k, phi, c, dt, stream);
 }
 
 int adjoint_filled(const nebo_field_t* lam_out, double* gk, const nebo_field_t* lam,
                    const nebo_field_t* phi, const nebo_field_t* k, const nebo_axis_coefs_t& c,
                    double dt, void* stream)
 {
-  Box3 B;
-  for (int d = 0; d < 3; ++d) B.n[d] = lam_out->extent[d] - 2;
-  B.nx = (B.n[0] + kTx - 1) / kTx;
-  B.ny = (B.n[1] + kTy - 1) / kTy;
-  B.nz = (B.n[2] + kZChunk - 1) / kZChunk;
-  B.zc = kZChunk;
-  const int nb = B.nx * B.ny * B.nz;
   const int X = lam_out->glob[0], XY = lam_out->glob[0] * lam_out->glob[1];
   // gk has k's shape: the same frame offset as k
   double* gko = gk + (frame_origin(k) - static_cast<double*>(k->values));
-  hipLaunchKernelGGL(adjoint_kernel, dim3(nb), dim3(kTx * kTy), 0, (hipStream_t)stream,
+  const nebo_limits_t lim = interior_of(lam_out);
+  const int cus = device_cu_count(lam_out->device);
+  auto groups = [&](int ty, int zc) {
+    return (long)((lim.hi[0] + kLanes - 1) / kLanes) * ((lim.hi[1] + ty - 1) / ty) * ((lim.hi[2] + zc - 1) / zc);
+  };
+  // By box size, us per step in a hipGraph of steps: column tiles of 4 rows and 8
+  // planes where the box gives a CU 28 waves of 2 rows and 8 planes (200^3: 103
+  // against 112 with 2 rows, 143 direct), 2 rows and 8 planes down to 6 such waves
+  // (128^3: 22.2 against 24.0), 4 planes to 2.5 (100x90x80: 13.2 against 14.1), and
+  // direct loads below, a wave per 2 planes of one row (64^3: 5.9; 27.3 with 16
+  // planes per wave, whose chain of planes set the time).
+  const long waves = groups(2, 8);
+  if (((long)XY + 2L * X + 2) * 8 < (1L << 31) && 2 * waves >= 5L * cus) {
+    const int ry = waves >= 28L * cus ? 4 : 2, zc = waves >= 6L * cus ? 8 : 4;
+    const auto fn = ry == 4 ? adjoint_column_kernel<4, 2, 0> : zc == 8 ? adjoint_column_kernel<2, 2, 0> : adjoint_column_kernel<2, 1, 0>;
+    const Tiles T = make_tiles(lim, kLanes, ry, zc);
+    hipLaunchKernelGGL(fn, dim3(T.nx * T.ny * T.nz), dim3(kLanes), 0, (hipStream_t)stream, frame_origin(lam_out), gko,
+                       frame_origin(lam), frame_origin(phi), frame_origin(k), T, zc, X, XY, c, dt);
+    const int rc = check_hip(hipGetLastError(), kCtx);
+    return rc ? rc : fill_thin_ghosts(lam_out, stream);
+  }
+  const Box3 B = make_box(lim.hi, kTx, 4, 2, 2);
+  const int nb = B.nx * B.ny * B.nz;
+  hipLaunchKernelGGL(adjoint_kernel, dim3(nb), dim3(box_threads(B)), 0, (hipStream_t)stream,
                      frame_origin(lam_out), gko, frame_origin(lam), frame_origin(phi), frame_origin(k), B,
                      X, XY, c, dt);
-  int rc = check_hip(hipGetLastError(), kCtx);
-  if (rc) return rc;
-  return fill_ghosts_periodic(lam_out, stream);
+  const int rc = check_hip(hipGetLastError(), kCtx);
+  return rc ? rc : fill_thin_ghosts(lam_out, stream);
 }
 
 }  // namespace

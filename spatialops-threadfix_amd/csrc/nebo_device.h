@@ -22,24 +22,30 @@ __device__ __forceinline__ int xcd_tile(int b, int nb)
   return x < r ? x * (q + 1) + k : r * (q + 1) + (x - r) * q + k;
 }
 
-// Tile grid over the n[0] x n[1] x n[2] interior of a periodic block: tiles of
-// 64 x TY columns marching ZC planes.
+// Tile grid over the n[0] x n[1] x n[2] interior of a periodic block: workgroups of
+// 64 columns x `rows` rows x zc planes, one wave per row and wz planes.
 struct Box3 {
   int n[3];
   int nx, ny, nz;  // tile counts
   int zc;          // planes per tile
+  int rows, wz;    // rows per tile, planes per wave
 };
 
-inline Box3 make_box(const int n[3], int tx, int ty, int zc)
+inline Box3 make_box(const int n[3], int tx, int ty, int zc, int wz)
 {
   Box3 B;
   for (int d = 0; d < 3; ++d) B.n[d] = n[d];
   B.zc = zc;
+  B.rows = ty;
+  const int zw = 16 / ty;   // at most 16 waves per workgroup
+  B.wz = (zc + zw - 1) / zw > wz ? (zc + zw - 1) / zw : wz;
   B.nx = (n[0] + tx - 1) / tx;
   B.ny = (n[1] + ty - 1) / ty;
   B.nz = (n[2] + zc - 1) / zc;
   return B;
 }
+
+inline int box_threads(const Box3& B) { return kLanes * B.rows * ((B.zc + B.wz - 1) / B.wz); }
 
 // interp(k)*grad(phi) on one face: (k_lo*i0 + k_hi*i1) * (p_lo*g0 + p_hi*g1)
 __device__ __forceinline__ double face_flux(double klo, double khi, double plo, double phi,
@@ -215,6 +221,54 @@ __device__ __forceinline__ PairGeom<RY> pair_geom(const Tiles& T, int X, int xw0
   else if (lane >= 32 && lane < 32 + RY) g.edge = off(xw0 + 2 * kLanes, min(y0 + lane - 32, T.hi[1]));
   else g.edge = g.row[1];
   return g;
+}
+
+// Ghost images of a periodic block with one ghost layer per face, written by the
+// kernel that forms the values: a separate fill is strided passes over the faces
+// (11 us after a 14 us step at 128^3).  image_step(i, n, s) is the distance, in
+// strides s, from interior coordinate i to its image along an axis of n >= 2 cells (0:
+// none; an axis of one cell has two, and its launcher fills the ghosts afterwards).
+__device__ __forceinline__ int image_step(int i, int n, int s) { return i == 0 ? n * s : i == n - 1 ? -n * s : 0; }
+
+// put(offset, z) for each image of a cell: `offset` from the cell's place in its plane,
+// in the plane itself or (z) the plane's own image.  Few cells have any, so every
+// group of stores is behind a branch that whole waves skip.
+template <typename F>
+__device__ __forceinline__ void for_images(int xo, int yo, bool zi, F&& put)
+{
+  if (xo) put(xo, false);
+  if (yo) {
+    put(yo, false);
+    if (xo) put(xo + yo, false);
+  }
+  if (zi) {
+    put(0, true);
+    if (xo) put(xo, true);
+    if (yo) {
+      put(yo, true);
+      if (xo) put(xo + yo, true);
+    }
+  }
+}
+
+// The images of v, the value of interior cell (x, y, z) of a block of n cells at o.
+__device__ __forceinline__ void store_images(double* o, int x, int y, int z, const int* n, int X, int XY, double v)
+{
+  const long zo = image_step(z, n[2], 1) * (long)XY;
+  for_images(image_step(x, n[0], 1), image_step(y, n[1], X), zo != 0,
+             [&](int off, bool zi) { o[off + (zi ? zo : 0)] = v; });
+}
+
+// The images of a column lane's value at byte offset `off` of plane z (box T from 0,
+// byte steps xo and yo of its column and row), in the planes of `out`.
+template <int SP>
+__device__ __forceinline__ void store_column_images(double* out, const Tiles& T, int X, int XY, int z, uint32_t off,
+                                                    int xo, int yo, double v)
+{
+  const int zo = image_step(z, T.hi[2], 1);
+  const Rsrc own = plane_rsrc(plane_base(out, T, X, XY, z), X, XY);
+  const Rsrc img = plane_rsrc(plane_base(out, T, X, XY, z + zo), X, XY);
+  for_images(xo, yo, zo != 0, [&](int d, bool zi) { store_at<SP>(zi ? img : own, off + d, v); });
 }
 
 // Run f(integral_constant<int, I>) for I = 0, 1, ... in order (compile-time steps).

@@ -225,10 +225,13 @@ int launch_lapl_euler(const nebo_field_t* out, const nebo_field_t* phi,
                       const nebo_axis_coefs_t& c, double s, const nebo_limits_t& lim,
                       void* stream);
 
-// out = phi + dt*div(interp(k)*grad(phi)) over lim (the diffusion kernel's Euler form).
+// out = phi + dt*div(interp(k)*grad(phi)) over the interior of one-ghost periodic
+// fields (the diffusion kernel's Euler form), and out's ghosts.
 int launch_diffusion_euler(const nebo_field_t* out, const nebo_field_t* k, const nebo_field_t* phi,
-                           const nebo_axis_coefs_t& c, double dt, const nebo_limits_t& lim,
-                           void* stream);
+                           const nebo_axis_coefs_t& c, double dt, void* stream);
+// After a kernel that writes the ghost images of f's cells: fills f's ghosts where an
+// axis has one cell, whose two images per axis such kernels leave out.
+int fill_thin_ghosts(const nebo_field_t* f, void* stream);
 // Periodic copy-fill of every allocated ghost layer of f.
 int fill_ghosts_periodic(const nebo_field_t* f, void* stream);
 

@@ -8,7 +8,7 @@
 // is evaluated by the generic evaluator (stencil folds of NeboStencils.h:407-448,
 // the first-true-clause select of NeboCond.h:408-412), so it is bit-identical to
 // nebo_assign of that stage expression.  Periodicity enters through one ghost
-// layer holding the wrapped interior; every stage refills its output's ghosts.
+// layer holding the wrapped interior; every stage writes its output's ghosts too.
 //
 // Transpose of a stage, for adjoint a and w_d = D_d^T a on the faces of axis d:
 //   R_s^T a    = sum_d G_d^T(kf_d .* w_d) - sum_d U_d^T(u_d .* w_d)
@@ -32,7 +32,6 @@ namespace nebo {
 namespace {
 
 constexpr int kTx = 64;
-constexpr int kTy = 4;
 constexpr int kZChunk = 16;
 const char* kCtx = "Nebo Transport";
 
@@ -51,6 +50,12 @@ Coefs3 coefs3(const nebo_axis_coefs_t& c)
   return r;
 }
 
+// Whether a column kernel writes its output's ghost images: the one-wave tiles of
+// small boxes do; the 128 x 8 tile of large ones leaves them to a fill, since its
+// stores wait behind the branches (512^3, three stages: 4191 us with images, 4137
+// with fills of one launch, 4149 with fills of three).
+constexpr bool column_images(int w, int nw) { return w * nw == 1; }
+
 // upwinded convective flux on one face: cond(u > 0, s_lo)(s_hi) * u
 __device__ __forceinline__ double conv_face(double u, double s_lo, double s_hi)
 {
@@ -58,7 +63,7 @@ __device__ __forceinline__ double conv_face(double u, double s_lo, double s_hi)
 }
 
 template <int STAGE>
-__global__ __launch_bounds__(kTx * kTy) void transport_stage_kernel(
+__global__ __launch_bounds__(1024) void transport_stage_kernel(
     double* __restrict__ out, const double* __restrict__ pn, const double* __restrict__ s,
     const double* __restrict__ k, const double* __restrict__ ux, const double* __restrict__ uy,
     const double* __restrict__ uz, Box3 B, int X, int XY, Coefs3 C, double dt)
@@ -69,10 +74,12 @@ __global__ __launch_bounds__(kTx * kTy) void transport_stage_kernel(
   const int ty = rest % B.ny;
   const int tz = rest / B.ny;
   const int x = tx * kTx + (threadIdx.x & (kTx - 1));
-  const int y = ty * kTy + (threadIdx.x / kTx);
+  const int wave = threadIdx.x / kTx;
+  const int y = ty * B.rows + wave % B.rows;
   if (x >= B.n[0] || y >= B.n[1]) return;
-  const int z0 = tz * B.zc;
-  const int z1 = min(z0 + B.zc, B.n[2]);
+  const int z0 = tz * B.zc + wave / B.rows * B.wz;
+  const int z1 = min(min(z0 + B.wz, (tz + 1) * B.zc), B.n[2]);
+  if (z0 >= z1) return;
   const AxisC cx = C.a[0], cy = C.a[1], cz = C.a[2];
 
   int i = x + X * y + XY * z0;
@@ -87,7 +94,7 @@ __global__ __launch_bounds__(kTx * kTy) void transport_stage_kernel(
     const double szp = s[i + XY], kzp = k[i + XY], uzh = uz[i + XY];
     const double sxm = s[i - 1], sxp = s[i + 1], kxm = k[i - 1], kxp = k[i + 1];
     const double sym = s[i - X], syp = s[i + X], kym = k[i - X], kyp = k[i + X];
-    const double uxl = ux[i], uxh = ux[i + 1], uyl = uy[i], uyh = uy[i + X];
+    const double uxl = ux[i], uxh = ux[i + 1], uyl = uy[i], uyh = uy[i + X], pnc = pn[i];
     const double fx = face_flux(kxm, kc, sxm, sc, cx.i0, cx.i1, cx.g0, cx.g1) * cx.d0 +
                       face_flux(kc, kxp, sc, sxp, cx.i0, cx.i1, cx.g0, cx.g1) * cx.d1;
     const double fy = face_flux(kym, kc, sym, sc, cy.i0, cy.i1, cy.g0, cy.g1) * cy.d0 +
@@ -100,10 +107,11 @@ __global__ __launch_bounds__(kTx * kTy) void transport_stage_kernel(
     const double vz = vz_lo * cz.d0 + vz_hi * cz.d1;
     const double R = ((fx + fy) + fz) - ((vx + vy) + vz);
     double v;
-    if constexpr (STAGE == 1) v = pn[i] + dt * R;
-    else if constexpr (STAGE == 2) v = 0.75 * pn[i] + 0.25 * (sc + dt * R);
-    else v = (1.0 / 3.0) * pn[i] + (2.0 / 3.0) * (sc + dt * R);
+    if constexpr (STAGE == 1) v = pnc + dt * R;
+    else if constexpr (STAGE == 2) v = 0.75 * pnc + 0.25 * (sc + dt * R);
+    else v = (1.0 / 3.0) * pnc + (2.0 / 3.0) * (sc + dt * R);
     out[i] = v;
+    store_images(&out[i], x, y, z, B.n, X, XY, v);
     sc = szp;
     kc = kzp;
     fz_lo = fz_hi;
@@ -124,8 +132,8 @@ __global__ __launch_bounds__(kTx * kTy) void transport_stage_kernel(
 // each plane's base (launcher: plane sizes below 2^31 bytes).  A plane slot is
 // 32 doubles, so the kernel takes the register file of one wave per SIMD (two
 // with loads one plane ahead): one 4-wave workgroup per CU, no spills.
-template <int STAGE, int W, int NW, int RY, int PF>
-__global__ __launch_bounds__(kLanes * W * NW) __attribute__((amdgpu_waves_per_eu(1, PF >= 2 ? 1 : 2)))
+template <int STAGE, int W, int NW, int RY, int PF, int SP = 2>
+__global__ __launch_bounds__(kLanes * W * NW) __attribute__((amdgpu_waves_per_eu(1, RY < 4 ? 4 : PF >= 2 ? 1 : 2)))
 void transport_column_kernel(
     double* __restrict__ out, const double* __restrict__ pn, const double* __restrict__ s,
     const double* __restrict__ k, const double* __restrict__ ux, const double* __restrict__ uy,
@@ -242,7 +250,12 @@ void transport_column_kernel(
         else v = (1.0 / 3.0) * C0.pn[j] + (2.0 / 3.0) * (sc + dt * R);
         fz[j] = fz_hi;
         vz[j] = vz_hi;
-        if (xin && y0 + j < T.hi[1]) store_nt_at(ob, g.row[j + 1], v);
+        if (xin && y0 + j < T.hi[1]) {
+          store_at<SP>(ob, g.row[j + 1], v);
+          if constexpr (column_images(W, NW))
+            store_column_images<SP>(out, T, X, XY, z, g.row[j + 1], image_step(x, T.hi[0], 8),
+                                    image_step(y0 + j, T.hi[1], 8 * X), v);
+        }
       }
       S[jj] = load(min(z + NS, z1));   // plane z is consumed: its slot takes z+NS
     }
@@ -280,7 +293,7 @@ __device__ __forceinline__ AdjCell adj_cell(const AdjFace& lo, const AdjFace& hi
 }
 
 template <int STAGE>
-__global__ __launch_bounds__(kTx * kTy) void transport_adjoint_kernel(
+__global__ __launch_bounds__(1024) void transport_adjoint_kernel(
     double* __restrict__ out, double* __restrict__ acc_out, double* __restrict__ gk,
     const double* __restrict__ a, const double* __restrict__ acc_in, const double* __restrict__ s,
     const double* __restrict__ k, const double* __restrict__ ux, const double* __restrict__ uy,
@@ -292,17 +305,20 @@ __global__ __launch_bounds__(kTx * kTy) void transport_adjoint_kernel(
   const int ty = rest % B.ny;
   const int tz = rest / B.ny;
   const int x = tx * kTx + (threadIdx.x & (kTx - 1));
-  const int y = ty * kTy + (threadIdx.x / kTx);
+  const int wave = threadIdx.x / kTx;
+  const int y = ty * B.rows + wave % B.rows;
   if (x >= B.n[0] || y >= B.n[1]) return;
-  const int z0 = tz * B.zc;
-  const int z1 = min(z0 + B.zc, B.n[2]);
+  const int z0 = tz * B.zc + wave / B.rows * B.wz;
+  const int z1 = min(min(z0 + B.wz, (tz + 1) * B.zc), B.n[2]);
+  if (z0 >= z1) return;
   const AxisC cx = C.a[0], cy = C.a[1], cz = C.a[2];
 
   int i = x + X * y + XY * z0;
   double ac = a[i], sc = s[i], kc = k[i];
   AdjFace zlo = adj_face(a[i - XY], ac, s[i - XY], sc, k[i - XY], kc, uz[i], cz);
   for (int z = z0; z < z1; ++z, i += XY) {
-    const double az = a[i + XY], szp = s[i + XY], kzp = k[i + XY];
+    const double az = a[i + XY], szp = s[i + XY], kzp = k[i + XY], gc = gk[i];
+    const double ain = STAGE == 3 ? 0.0 : acc_in[i];   // stage 3 reads no acc_in
     const AdjFace xlo = adj_face(a[i - 1], ac, s[i - 1], sc, k[i - 1], kc, ux[i], cx);
     const AdjFace xhi = adj_face(ac, a[i + 1], sc, s[i + 1], kc, k[i + 1], ux[i + 1], cx);
     const AdjFace ylo = adj_face(a[i - X], ac, s[i - X], sc, k[i - X], kc, uy[i], cy);
@@ -311,16 +327,12 @@ __global__ __launch_bounds__(kTx * kTy) void transport_adjoint_kernel(
     const AdjCell ex = adj_cell(xlo, xhi, cx), ey = adj_cell(ylo, yhi, cy), ez = adj_cell(zlo, zhi, cz);
     const double rt = ((ex.A + ey.A) + ez.A) - ((ex.V + ey.V) + ez.V);
     const double Xv = ac + dt * rt;
-    if constexpr (STAGE == 3) {
-      out[i] = cs * Xv;
-      acc_out[i] = (1.0 / 3.0) * ac;
-    } else if constexpr (STAGE == 2) {
-      out[i] = cs * Xv;
-      acc_out[i] = acc_in[i] + 0.75 * ac;
-    } else {
-      out[i] = acc_in[i] + Xv;
-    }
-    gk[i] = gk[i] + cdt * ((ex.B + ey.B) + ez.B);
+    const double v = STAGE == 1 ? ain + Xv : cs * Xv;
+    out[i] = v;
+    store_images(&out[i], x, y, z, B.n, X, XY, v);
+    if constexpr (STAGE == 3) acc_out[i] = (1.0 / 3.0) * ac;
+    else if constexpr (STAGE == 2) acc_out[i] = ain + 0.75 * ac;
+    gk[i] = gc + cdt * ((ex.B + ey.B) + ez.B);
     ac = az;
     sc = szp;
     kc = kzp;
@@ -333,8 +345,8 @@ __global__ __launch_bounds__(kTx * kTy) void transport_adjoint_kernel(
 // the face velocities as in the stage kernel, acc_in and g_k on the lane's rows.
 // Every cell is evaluated in transport_adjoint_kernel's order (bit-identical);
 // g_k is read before its cell is written and read by no other cell.
-template <int STAGE, int W, int NW, int RY, int PF>
-__global__ __launch_bounds__(kLanes * W * NW) __attribute__((amdgpu_waves_per_eu(1, PF >= 2 ? 1 : 2)))
+template <int STAGE, int W, int NW, int RY, int PF, int SP = 2>
+__global__ __launch_bounds__(kLanes * W * NW) __attribute__((amdgpu_waves_per_eu(1, RY < 4 ? 4 : PF >= 2 ? 1 : 2)))
 void transport_adjoint_column_kernel(
     double* __restrict__ out, double* __restrict__ acc_out, double* __restrict__ gk,
     const double* __restrict__ a, const double* __restrict__ acc_in, const double* __restrict__ s,
@@ -448,16 +460,16 @@ void transport_adjoint_column_kernel(
         zlo[j] = zhi;
         if (xin && y0 + j < T.hi[1]) {
           const uint32_t o = g.row[j + 1];
-          if constexpr (STAGE == 3) {
-            store_nt_at(ob, o, cs * Xv);
-            store_nt_at(plane_rsrc(plane_base(acc_out, T, X, XY, z), X, XY), o, (1.0 / 3.0) * ac);
-          } else if constexpr (STAGE == 2) {
-            store_nt_at(ob, o, cs * Xv);
-            store_nt_at(plane_rsrc(plane_base(acc_out, T, X, XY, z), X, XY), o, C0.ain[j] + 0.75 * ac);
-          } else {
-            store_nt_at(ob, o, C0.ain[j] + Xv);
-          }
-          store_nt_at(gb, o, gnew);
+          const double v = STAGE == 1 ? C0.ain[j] + Xv : cs * Xv;
+          store_at<SP>(ob, o, v);
+          if constexpr (STAGE == 3)
+            store_at<SP>(plane_rsrc(plane_base(acc_out, T, X, XY, z), X, XY), o, (1.0 / 3.0) * ac);
+          else if constexpr (STAGE == 2)
+            store_at<SP>(plane_rsrc(plane_base(acc_out, T, X, XY, z), X, XY), o, C0.ain[j] + 0.75 * ac);
+          store_at<SP>(gb, o, gnew);
+          if constexpr (column_images(W, NW))
+            store_column_images<SP>(out, T, X, XY, z, g.row[j + 1], image_step(x, T.hi[0], 8),
+                                    image_step(y0 + j, T.hi[1], 8 * X), v);
         }
       }
       S[jj] = load(min(z + NS, z1));
@@ -476,7 +488,7 @@ struct Operands {
   const nebo_field_t* k;
 };
 
-// Stage schedule: 0 chosen by box size; 1 direct (64 x 4 columns); 2 column
+// Stage schedule: 0 chosen by box size; 1 direct; 2 column
 // tiles with loads 2 planes ahead; 3 column tiles with loads 1 plane ahead.
 // g_zchunk: planes per workgroup, 0 for the schedule's default.
 std::atomic<int> g_schedule{0};
@@ -484,78 +496,133 @@ std::atomic<int> g_zchunk{0};
 
 constexpr int kColW = 2, kColNW = 2, kColRY = 4;   // column tiles of 128 x 8 cells
 
-// Schedule and z chunk of a stage over an n[0] x n[1] x n[2] interior.  By box
-// size: column tiles (loads 1 plane ahead) with the longest chunk (512 .. 64
-// planes) that gives every CU a workgroup, as the stencil kernels do, else the
-// direct schedule.
-void stage_schedule(const nebo_field_t* f, int* sched, int* zc)
+// How a stage (or its transpose) runs over a box: direct loads (sched 1: workgroups of
+// 64 columns x rows x zc planes, a wave per row and wz planes) or column tiles (2, 3:
+// loads 2 or 1 planes ahead) of 128 x 8 cells, or of one wave with ry rows per lane.
+struct StagePlan {
+  int sched, zc;
+  int rows, wz;   // direct
+  int ry;         // column: rows per lane of a one-wave tile, 0: the 128 x 8 tile
+  bool nt;        // one-wave tiles: nontemporal stores
+};
+
+// By box size, unless nebo_transport_tune set a schedule (the 128 x 8 tile's or the
+// direct one; its z chunk applies to either).  us per stage of 8 steps' worth of
+// launches in a hipGraph, stage 2 and its transpose:
+//  1. the 128 x 8 tile with loads 1 plane ahead and the longest chunk (512 .. 64
+//     planes) that gives every CU a workgroup, where the box fills two thirds of the
+//     cells its rounds of workgroups hold (256^3: 197 and 326);
+//  2. boxes that give a CU 28 waves of 2 rows x 8 planes: one-wave tiles of 4 rows
+//     and 8 planes (200^3: 111 and 177 against 132 and 256 direct);
+//  3. the transpose on smaller boxes, down to 2.5 such waves: one-wave tiles of 2 rows
+//     and 8 planes, 4 planes below 6 waves (160^3: 78 against 127 direct, 112x96x80:
+//     18.6 against 22.3); the stage, with fewer fields, is as fast on direct loads
+//     there (160^3 44.3 against 42.1, 112x96x80 13.5 against 12.3);
+//  4. direct loads: a wave per 4 planes of one row, two rows and 16 planes per
+//     workgroup; where that leaves a CU fewer than 8 waves, per 2 planes, one row per
+//     workgroup (64^3: 5.0 and 8.7 against 22.9 and 28.6 with 16 planes per wave, whose
+//     chain of planes set the time); and workgroups of 4 rows and 2 planes where even
+//     those leave CUs without one (32^3: 3.7 and 5.5 against 23.1 and 26.8).
+// One-wave tiles store nontemporally where the pass's fields (7, or 11) do not fit the
+// 256 MB memory-side cache (transpose at 160^3, 374 MB: 78 against 92; at 128^3, 193
+// MB: 36.3 against 34.3).
+StagePlan stage_plan(const nebo_field_t* f, bool transpose)
 {
   const int n[3] = {f->extent[0] - 2, f->extent[1] - 2, f->extent[2] - 2};
-  *sched = g_schedule.load();
+  StagePlan P{g_schedule.load(), 0, 2, 4, 0, false};
   int auto_zc = 64;
-  if (*sched == 0) {
-    *sched = 1;
-    const long cols = (long)((n[0] + kLanes * kColW - 1) / (kLanes * kColW)) *
-                      ((n[1] + kColRY * kColNW - 1) / (kColRY * kColNW));
-    const int cus = device_cu_count(f->device);
-    for (int c : {512, 256, 128, 64})
-      if (cols * ((n[2] + c - 1) / c) >= cus) {
-        *sched = 3;   // loads 1 plane ahead: 1388 us per stage at 512^3 on MI355X, 2 planes 1413, direct 1797
-        auto_zc = c;
-        break;
-      }
-  }
+  auto groups = [&](int tx, int ty, int zc) {
+    return (long)((n[0] + tx - 1) / tx) * ((n[1] + ty - 1) / ty) * ((n[2] + zc - 1) / zc);
+  };
   // the column schedule's 32-bit plane offsets
   const long X = f->glob[0], XY = (long)f->glob[0] * f->glob[1];
-  if (*sched >= 2 && (XY + 2 * X + 2) * 8 >= (1L << 31)) *sched = 1;
-  *zc = g_zchunk.load() > 0 ? g_zchunk.load() : *sched == 1 ? kZChunk : auto_zc;
+  const bool columns = (XY + 2 * X + 2) * 8 < (1L << 31);
+  const int cus = device_cu_count(f->device);
+  if (P.sched == 0) {
+    P.sched = 1;
+    const int tx = kLanes * kColW, ty = kColRY * kColNW;
+    const double cells = (double)n[0] * n[1] * n[2];
+    for (int c : {512, 256, 128, 64}) {
+      const long g = groups(tx, ty, c);
+      if (g < cus) continue;
+      if (cells >= 0.66 * (double)((g + cus - 1) / cus * cus) * tx * ty * c) {
+        P.sched = 3;   // loads 1 plane ahead: 1388 us per stage at 512^3 on MI355X, 2 planes 1413, direct 1797
+        auto_zc = c;
+      }
+      break;
+    }
+    const long waves = groups(kLanes, 2, 8);
+    if (P.sched == 1 && columns && (waves >= 28L * cus || (transpose && 2 * waves >= 5L * cus))) {
+      P.sched = 3;
+      P.ry = waves >= 28L * cus ? 4 : 2;
+      auto_zc = waves >= 6L * cus ? 8 : 4;
+      P.nt = (transpose ? 11 : 7) * 8.0 * (double)field_npts(f) > 256.0 * (1 << 20);
+    }
+  }
+  if (P.sched >= 2 && !columns) P.sched = 1;
+  P.zc = g_zchunk.load() > 0 ? g_zchunk.load() : P.sched == 1 ? kZChunk : auto_zc;
+  if (P.sched == 1 && g_schedule.load() == 0 && g_zchunk.load() == 0 && groups(kTx, 1, 4) < 8L * cus) {
+    P.rows = 1;
+    P.wz = 2;
+    if (groups(kTx, 1, kZChunk) < cus) {
+      P.rows = 4;
+      P.zc = 2;
+    }
+  }
+  return P;
 }
 
 using ColumnFn = void (*)(double*, const double*, const double*, const double*, const double*, const double*,
                           const double*, Tiles, int, int, int, Coefs3, double);
 
-ColumnFn column_fn(int stage, int pf)
+template <int W, int NW, int RY, int PF, int SP>
+ColumnFn column_of(int stage)
 {
-  static const ColumnFn t[2][3] = {
-      {transport_column_kernel<1, kColW, kColNW, kColRY, 2>, transport_column_kernel<2, kColW, kColNW, kColRY, 2>,
-       transport_column_kernel<3, kColW, kColNW, kColRY, 2>},
-      {transport_column_kernel<1, kColW, kColNW, kColRY, 1>, transport_column_kernel<2, kColW, kColNW, kColRY, 1>,
-       transport_column_kernel<3, kColW, kColNW, kColRY, 1>}};
-  return t[pf == 2 ? 0 : 1][stage - 1];
+  return stage == 1   ? transport_column_kernel<1, W, NW, RY, PF, SP>
+         : stage == 2 ? transport_column_kernel<2, W, NW, RY, PF, SP>
+                      : transport_column_kernel<3, W, NW, RY, PF, SP>;
 }
+
+ColumnFn column_fn(int stage, const StagePlan& P)
+{
+  if (P.ry == 4) return P.nt ? column_of<1, 1, 4, 1, 2>(stage) : column_of<1, 1, 4, 1, 0>(stage);
+  return P.sched == 2 ? column_of<kColW, kColNW, kColRY, 2, 2>(stage) : column_of<kColW, kColNW, kColRY, 1, 2>(stage);
+}
+
+Tiles column_tiles(const nebo_field_t* f, const StagePlan& P)
+{
+  return P.ry ? make_tiles(interior_of(f), kLanes, P.ry, P.zc)
+              : make_tiles(interior_of(f), kLanes * kColW, kColRY * kColNW, P.zc);
+}
+
+unsigned column_threads(const StagePlan& P) { return P.ry ? kLanes : kLanes * kColW * kColNW; }
 
 int launch_stage(const nebo_field_t* out, const nebo_field_t* pn, const nebo_field_t* s,
                  const Operands& o, const nebo_axis_coefs_t& c, double dt, int stage, void* stream)
 {
-  int sched = 1, zc = kZChunk;
-  stage_schedule(out, &sched, &zc);
+  const StagePlan P = stage_plan(out, false);
   const int X = out->glob[0], XY = out->glob[0] * out->glob[1];
   const double* sp = frame_origin(stage == 1 ? pn : s);
-  if (sched == 1) {
+  if (P.sched == 1) {
     const int n[3] = {out->extent[0] - 2, out->extent[1] - 2, out->extent[2] - 2};
-    const Box3 B = make_box(n, kTx, kTy, zc);
+    const Box3 B = make_box(n, kTx, P.rows, P.zc, P.wz);
     const int nb = B.nx * B.ny * B.nz;
     auto fn = stage == 1 ? transport_stage_kernel<1> : stage == 2 ? transport_stage_kernel<2>
                                                                   : transport_stage_kernel<3>;
-    hipLaunchKernelGGL(fn, dim3(nb), dim3(kTx * kTy), 0, (hipStream_t)stream, frame_origin(out),
+    hipLaunchKernelGGL(fn, dim3(nb), dim3(box_threads(B)), 0, (hipStream_t)stream, frame_origin(out),
                        frame_origin(pn), sp, frame_origin(o.k), frame_origin(&o.u[0]), frame_origin(&o.u[1]),
                        frame_origin(&o.u[2]), B, X, XY, coefs3(c), dt);
   } else {
-    nebo_limits_t L;
-    for (int d = 0; d < 3; ++d) {
-      L.lo[d] = 0;
-      L.hi[d] = out->extent[d] - 2;
-    }
-    const Tiles T = make_tiles(L, kLanes * kColW, kColRY * kColNW, zc);
+    const Tiles T = column_tiles(out, P);
     const long nb = (long)T.nx * T.ny * T.nz;
-    hipLaunchKernelGGL(column_fn(stage, sched == 2 ? 2 : 1), dim3((unsigned)nb), dim3(kLanes * kColW * kColNW), 0,
+    hipLaunchKernelGGL(column_fn(stage, P), dim3((unsigned)nb), dim3(column_threads(P)), 0,
                        (hipStream_t)stream, frame_origin(out), frame_origin(pn), sp, frame_origin(o.k),
-                       frame_origin(&o.u[0]), frame_origin(&o.u[1]), frame_origin(&o.u[2]), T, zc, X, XY,
+                       frame_origin(&o.u[0]), frame_origin(&o.u[1]), frame_origin(&o.u[2]), T, P.zc, X, XY,
                        coefs3(c), dt);
   }
-  int rc = check_hip(hipGetLastError(), kCtx);
+  const int rc = check_hip(hipGetLastError(), kCtx);
   if (rc) return rc;
-  return fill_ghosts_periodic(out, stream);
+  return P.sched == 1 || P.ry ? fill_thin_ghosts(out, stream) : fill_ghosts_periodic(out, stream);
 }
 
 double stage_weight(int stage) { return stage == 3 ? 2.0 / 3.0 : stage == 2 ? 0.25 : 1.0; }
@@ -564,24 +631,27 @@ using AdjColumnFn = void (*)(double*, double*, double*, const double*, const dou
                              const double*, const double*, const double*, const double*, Tiles, int, int, int,
                              Coefs3, double, double, double);
 
-AdjColumnFn adjoint_column_fn(int stage, int pf)
+template <int W, int NW, int RY, int PF, int SP>
+AdjColumnFn adjoint_column_of(int stage)
 {
-  static const AdjColumnFn t[2][3] = {
-      {transport_adjoint_column_kernel<1, kColW, kColNW, kColRY, 2>,
-       transport_adjoint_column_kernel<2, kColW, kColNW, kColRY, 2>,
-       transport_adjoint_column_kernel<3, kColW, kColNW, kColRY, 2>},
-      {transport_adjoint_column_kernel<1, kColW, kColNW, kColRY, 1>,
-       transport_adjoint_column_kernel<2, kColW, kColNW, kColRY, 1>,
-       transport_adjoint_column_kernel<3, kColW, kColNW, kColRY, 1>}};
-  return t[pf == 2 ? 0 : 1][stage - 1];
+  return stage == 1   ? transport_adjoint_column_kernel<1, W, NW, RY, PF, SP>
+         : stage == 2 ? transport_adjoint_column_kernel<2, W, NW, RY, PF, SP>
+                      : transport_adjoint_column_kernel<3, W, NW, RY, PF, SP>;
+}
+
+AdjColumnFn adjoint_column_fn(int stage, const StagePlan& P)
+{
+  if (P.ry == 4) return P.nt ? adjoint_column_of<1, 1, 4, 1, 2>(stage) : adjoint_column_of<1, 1, 4, 1, 0>(stage);
+  if (P.ry == 2) return P.nt ? adjoint_column_of<1, 1, 2, 1, 2>(stage) : adjoint_column_of<1, 1, 2, 1, 0>(stage);
+  return P.sched == 2 ? adjoint_column_of<kColW, kColNW, kColRY, 2, 2>(stage)
+                      : adjoint_column_of<kColW, kColNW, kColRY, 1, 2>(stage);
 }
 
 int launch_adjoint(const nebo_field_t* out, double* acc_out, double* gk, const nebo_field_t* a,
                    const double* acc_in, const nebo_field_t* s, const Operands& o,
                    const nebo_axis_coefs_t& c, double dt, int stage, void* stream)
 {
-  int sched = 1, zc = kZChunk;
-  stage_schedule(out, &sched, &zc);
+  const StagePlan P = stage_plan(out, true);
   const int X = out->glob[0], XY = out->glob[0] * out->glob[1];
   // acc and gk are plain blocks with the field's shape: offset them like the field
   const std::ptrdiff_t off = frame_origin(out) - static_cast<double*>(out->values);
@@ -589,31 +659,25 @@ int launch_adjoint(const nebo_field_t* out, double* acc_out, double* gk, const n
   const double cdt = cs * dt;
   double* acc_o = acc_out ? acc_out + off : nullptr;
   const double* acc_i = acc_in ? acc_in + off : nullptr;
-  if (sched == 1) {
+  if (P.sched == 1) {
     const int n[3] = {out->extent[0] - 2, out->extent[1] - 2, out->extent[2] - 2};
-    const Box3 B = make_box(n, kTx, kTy, zc);
+    const Box3 B = make_box(n, kTx, P.rows, P.zc, P.wz);
     const int nb = B.nx * B.ny * B.nz;
     auto fn = stage == 1 ? transport_adjoint_kernel<1> : stage == 2 ? transport_adjoint_kernel<2>
                                                                     : transport_adjoint_kernel<3>;
-    hipLaunchKernelGGL(fn, dim3(nb), dim3(kTx * kTy), 0, (hipStream_t)stream, frame_origin(out), acc_o, gk + off,
+    hipLaunchKernelGGL(fn, dim3(nb), dim3(box_threads(B)), 0, (hipStream_t)stream, frame_origin(out), acc_o, gk + off,
                        frame_origin(a), acc_i, frame_origin(s), frame_origin(o.k), frame_origin(&o.u[0]),
                        frame_origin(&o.u[1]), frame_origin(&o.u[2]), B, X, XY, coefs3(c), dt, cs, cdt);
   } else {
-    nebo_limits_t L;
-    for (int d = 0; d < 3; ++d) {
-      L.lo[d] = 0;
-      L.hi[d] = out->extent[d] - 2;
-    }
-    const Tiles T = make_tiles(L, kLanes * kColW, kColRY * kColNW, zc);
+    const Tiles T = column_tiles(out, P);
     const long nb = (long)T.nx * T.ny * T.nz;
-    hipLaunchKernelGGL(adjoint_column_fn(stage, sched == 2 ? 2 : 1), dim3((unsigned)nb),
-                       dim3(kLanes * kColW * kColNW), 0, (hipStream_t)stream, frame_origin(out), acc_o, gk + off,
+    hipLaunchKernelGGL(adjoint_column_fn(stage, P), dim3((unsigned)nb), dim3(column_threads(P)), 0, (hipStream_t)stream, frame_origin(out), acc_o, gk + off,
                        frame_origin(a), acc_i, frame_origin(s), frame_origin(o.k), frame_origin(&o.u[0]),
-                       frame_origin(&o.u[1]), frame_origin(&o.u[2]), T, zc, X, XY, coefs3(c), dt, cs, cdt);
+                       frame_origin(&o.u[1]), frame_origin(&o.u[2]), T, P.zc, X, XY, coefs3(c), dt, cs, cdt);
   }
-  int rc = check_hip(hipGetLastError(), kCtx);
+  const int rc = check_hip(hipGetLastError(), kCtx);
   if (rc) return rc;
-  return fill_ghosts_periodic(out, stream);
+  return P.sched == 1 || P.ry ? fill_thin_ghosts(out, stream) : fill_ghosts_periodic(out, stream);
 }
 
 // k, u[0..2] and every state field share ref's periodic window.
@@ -659,10 +723,9 @@ extern "C" int nebo_transport_schedule(const nebo_field_t* field, int32_t* sched
 {
   clear_error();
   if (!field) return set_error(NEBO_ERR_INVALID, kCtx, "null argument");
-  int sched = 1, zc = kZChunk;
-  stage_schedule(field, &sched, &zc);
-  if (schedule) *schedule = sched;
-  if (zchunk) *zchunk = zc;
+  const StagePlan P = stage_plan(field, false);
+  if (schedule) *schedule = P.sched;
+  if (zchunk) *zchunk = P.zc;
   return NEBO_OK;
 }
 
