@@ -753,7 +753,12 @@ constexpr int prefetch_planes(const TileShape& sh)
          : sh.variant == 8                       ? 4
                                                  : 2;
 }
-// Cache policy of a column tile's stores (2 nontemporal, 0 write-back).
+// Cache policy of a column tile's stores (2 nontemporal, 0 write-back).  The Euler
+// step's one-wave tiles always write back: the next step reads what this one wrote, from
+// the memory-side cache where it fits (steps in a row, 160^3 24.7 us against 32.9,
+// 200^3 44.7 against 59.1, 300^3 172 against 182).  An assignment's result may not be
+// read at once, and its nontemporal stores leave that cache to the operands (160^3,
+// three sets of fields in turn: 21.3 us against 30.6).
 constexpr int store_policy(const TileShape& sh) { return sh.variant == 9 ? 0 : 2; }
 constexpr int stacked_waves(const TileShape& sh) { return sh.ty / rows_per_lane(sh); }
 
@@ -790,7 +795,7 @@ constexpr DivkFn divk_fn()
                                 prefetch_planes(sh)>;
   else if constexpr (sh.variant >= 3)
     return divkgrad_column_kernel<FORM, sh.tx / kTx, stacked_waves(sh), rows_per_lane(sh), sh.zc, sh.variant != 3,
-                                  prefetch_planes(sh), store_policy(sh)>;
+                                  prefetch_planes(sh), FORM == 2 && tile_geometry(sh).threads == kTx ? 0 : store_policy(sh)>;
   else return divkgrad_staged_kernel<FORM, sh.ty, sh.zc, sh.variant>;
 }
 

@@ -503,7 +503,7 @@ struct StagePlan {
   int sched, zc;
   int rows, wz;   // direct
   int ry;         // column: rows per lane of a one-wave tile, 0: the 128 x 8 tile
-  bool nt;        // one-wave tiles: nontemporal stores
+  bool nt;        // one-wave tiles of 2 rows: nontemporal stores
 };
 
 // By box size, unless nebo_transport_tune set a schedule (the 128 x 8 tile's or the
@@ -523,9 +523,11 @@ struct StagePlan {
 //     workgroup (64^3: 5.0 and 8.7 against 22.9 and 28.6 with 16 planes per wave, whose
 //     chain of planes set the time); and workgroups of 4 rows and 2 planes where even
 //     those leave CUs without one (32^3: 3.7 and 5.5 against 23.1 and 26.8).
-// One-wave tiles store nontemporally where the pass's fields (7, or 11) do not fit the
-// 256 MB memory-side cache (transpose at 160^3, 374 MB: 78 against 92; at 128^3, 193
-// MB: 36.3 against 34.3).
+// One-wave tiles write back, for the next pass to read (trajectory gradients at 200^3
+// 4832 us against 4960, 300^3 14981 against 15251), but those of 2 rows store
+// nontemporally where the transpose's 11 fields do not fit the 256 MB memory-side cache
+// (160^3 2285 against 2321; the pass alone, 78 against 92; at 128^3, 193 MB, 36.3
+// against 34.3).
 StagePlan stage_plan(const nebo_field_t* f, bool transpose)
 {
   const int n[3] = {f->extent[0] - 2, f->extent[1] - 2, f->extent[2] - 2};
@@ -556,7 +558,7 @@ StagePlan stage_plan(const nebo_field_t* f, bool transpose)
       P.sched = 3;
       P.ry = waves >= 28L * cus ? 4 : 2;
       auto_zc = waves >= 6L * cus ? 8 : 4;
-      P.nt = (transpose ? 11 : 7) * 8.0 * (double)field_npts(f) > 256.0 * (1 << 20);
+      P.nt = P.ry == 2 && 11 * 8.0 * (double)field_npts(f) > 256.0 * (1 << 20);
     }
   }
   if (P.sched >= 2 && !columns) P.sched = 1;
@@ -585,7 +587,7 @@ ColumnFn column_of(int stage)
 
 ColumnFn column_fn(int stage, const StagePlan& P)
 {
-  if (P.ry == 4) return P.nt ? column_of<1, 1, 4, 1, 2>(stage) : column_of<1, 1, 4, 1, 0>(stage);
+  if (P.ry == 4) return column_of<1, 1, 4, 1, 0>(stage);
   return P.sched == 2 ? column_of<kColW, kColNW, kColRY, 2, 2>(stage) : column_of<kColW, kColNW, kColRY, 1, 2>(stage);
 }
 
@@ -641,7 +643,7 @@ AdjColumnFn adjoint_column_of(int stage)
 
 AdjColumnFn adjoint_column_fn(int stage, const StagePlan& P)
 {
-  if (P.ry == 4) return P.nt ? adjoint_column_of<1, 1, 4, 1, 2>(stage) : adjoint_column_of<1, 1, 4, 1, 0>(stage);
+  if (P.ry == 4) return adjoint_column_of<1, 1, 4, 1, 0>(stage);
   if (P.ry == 2) return P.nt ? adjoint_column_of<1, 1, 2, 1, 2>(stage) : adjoint_column_of<1, 1, 2, 1, 0>(stage);
   return P.sched == 2 ? adjoint_column_of<kColW, kColNW, kColRY, 2, 2>(stage)
                       : adjoint_column_of<kColW, kColNW, kColRY, 1, 2>(stage);
