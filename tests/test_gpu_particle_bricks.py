@@ -84,3 +84,34 @@ def test_dense_and_empty_bricks_together():
     mix = rng.permutation(30500)
     scatter(L, np.concatenate([a[0], b[0]])[mix], [np.concatenate([x, y])[mix] for x, y in zip(a[1], b[1])],
             np.concatenate([a[2], b[2]])[mix], (1.0, 0.5, 1.0, 0.5, 1.0, 0.5))
+
+
+@pytest.mark.parametrize("axes", [(0,), (1, 2), (0, 1, 2)])
+@pytest.mark.parametrize("edge,spacing", [((0.2, 1.5), (1.0, 1.0, 1.0)), ((1.0, 1.0), (1.0, 1.0, 1.0)),
+                                          ((2.5, 4.5), (0.3, 0.7, 1.1)), ((0.2, 2.0), (3e-151, 3e-151, 3e-151)),
+                                          ((0.2, 2.0), (1e140, 1e140, 1e140)), ((0.0, 0.0), (1.0, 1.0, 1.0))])
+def test_gather_of_every_span(axes, edge, spacing):
+    """CellToParticle of particles of up to three cells per axis and more, with faces on
+    cell faces, and with spacings whose products leave the range of the fast quotient."""
+    n = tuple(17 if a in axes else 1 for a in range(3))
+    L = nh.Layout.build(n, 1)
+    rng = np.random.default_rng(int(10 * edge[1]) + len(axes))
+    m = 3000
+    unit = rng.uniform(*edge, m)
+    size = unit * min(spacing[a] for a in axes)
+    coords = [None] * 3
+    for a in axes:
+        x = rng.uniform(-2.0, 19.0, m)
+        x[::3] = np.floor(x[::3]) + unit[::3] / 2      # the low face on a cell face
+        coords[a] = x * spacing[a]
+    geom = tuple(v for a in range(3) for v in ((spacing[a], 0.5 * spacing[a]) if a in axes else (-1.0, 0.0)))
+    cells = nh.Field.from_numpy(L, rng.standard_normal(L.npts), where="both")
+    op = P.CellToParticle(*geom)
+    op.set_coordinate_information(*[dev(c) for c in coords], dev(size))
+    skipped = torch.zeros(1, dtype=torch.int32, device="cuda:0")
+    out = op.apply_to_field(cells, torch.full((m,), 9.0, dtype=torch.float64, device="cuda:0"), skipped=skipped)
+    torch.cuda.synchronize()
+    with np.errstate(all="ignore"):
+        want = orc.cell_to_particle(cells, *coords, size, geom, m)
+    assert np.array_equal(out.cpu().numpy(), want, equal_nan=True)
+    assert skipped.item() > 0
