@@ -523,7 +523,8 @@ __global__ __launch_bounds__(kRowCols * kRowSegments) void scan_rows(uint32_t* _
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (r + u < r1) mine[(size_t)(r + u) * n_bricks] = at;
+      if (r + u >= r1) continue;   // past the part v repeats its last row
+      mine[(size_t)(r + u) * n_bricks] = at;
       at += v[u];
     }
   }

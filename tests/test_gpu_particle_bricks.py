@@ -46,6 +46,18 @@ def test_windows_that_end_inside_a_brick(n, npart):
     assert below > 0 or npart == 3
 
 
+# Blocks of counting particles (one per 1024, up to 512, or more where the bricks are
+# few), whose counts are summed in 64 parts: one row per part, a last part that is
+# full, cut, and empty, and parts longer than one batch of loads.
+@pytest.mark.parametrize("npart", [64 * 1024, 65 * 1024, 126 * 1024, 127 * 1024 - 5, 128 * 1024, 443 * 1024 - 7,
+                                   511 * 1024 + 1, 600 * 1024, 760 * 1024, 1500 * 1024])
+def test_counts_of_every_number_of_blocks(npart):
+    n = (50, 70, 36)
+    L = nh.Layout.build(n, 1)
+    rng = np.random.default_rng(npart)
+    scatter(L, *cloud(rng, npart, [(0.0, float(e)) for e in n], 0.2, 1.2, beyond=0.5), (1.0, 0.5, 1.0, 0.5, 1.0, 0.5))
+
+
 @pytest.mark.parametrize("edge", [0.0, 1.0, 6.5, 30.0])
 def test_particles_of_every_size(edge):
     """Cubes of no volume (0/0 in the reference too), of whole cells, wider than a
