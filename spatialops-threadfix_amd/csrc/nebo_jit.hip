@@ -32,6 +32,7 @@
 #include <hip/hiprtc.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <functional>
 #include <cstring>
@@ -574,6 +575,21 @@ bool select_ring(const VmProgram& P, ColumnPlan* cp, bool pairs)
   // lane and dropped planes against 4.52-4.55 with one column; div(k grad phi)
   // at 256^3 67.5 us with two columns and 2 rows as they are against 72.3-74.0
   // with its planes dropped).
+  // A family read on one x side over both rows and planes (filters, corners) keeps
+  // one column: the neighbours it shares leave no room for two (at 200^3, one
+  // column against two: a filter with a second field 58.3 us against 63.3, the
+  // eight corners of two fields 51.4 against 61.0), where rows or planes alone
+  // leave it (the 9-point squares of two fields 51.7 and 44.0).
+  for (int f = 0; f < cp->nf; ++f)
+    for (int right = 0; right < 2; ++right) {
+      int lo[2] = {2, 2}, hi[2] = {-2, -2};
+      for (int s = 0; s < kVmMaxLoads; ++s)
+        if (cp->fam[s] == f && cp->dx[s] != 0 && (cp->dx[s] > 0) == (right == 1)) {
+          lo[0] = std::min(lo[0], cp->dy[s]), hi[0] = std::max(hi[0], cp->dy[s]);
+          lo[1] = std::min(lo[1], cp->dz[s]), hi[1] = std::max(hi[1], cp->dz[s]);
+        }
+      pairs = pairs && !(hi[0] > lo[0] && hi[1] > lo[1]);
+    }
   cp->RY = 0;
   for (int pair = (pairs && cp->nf >= 2) ? 1 : 0; pair >= 0 && !cp->RY; --pair) {
     cp->pair = pair == 1;
@@ -728,8 +744,47 @@ std::string jit_column_source(const VmProgram& P, const SlotUse& u, const Column
   // return 0)
   auto zl = [&](int f) { return cp.zlo[f] + (cp.drop[f] ? 1 : 0); };
   auto nslots = [&](int f) { return cp.zhi[f] - zl(f) + 1 + cp.PF; };
+  // Shared neighbours.  Where a family's reads on one x side lie on several rows
+  // or planes (a 27-point filter), each value from the adjacent lane is wanted by
+  // several cells of the lane: it is formed once per row as its plane comes into
+  // use, and kept beside the ring until the last plane that reads it.  Formed at
+  // every read, these exchanges were two thirds of the filter's instructions (870
+  // per step of 4 cells, now 440) and bounded it: 180x150x130 44.5 -> 20.0 us,
+  // 256^3 107 -> 72.3, 300^3 322 -> 152, 512 x 512 x 256 347 -> 269.  A side read
+  // at one row and plane only (face
+  // gradients) has each value used once, and is exchanged where it is read.
+  struct Shared { bool on = false; int ylo = 2, yhi = -2, zlo = 2, zhi = -2; };
+  std::vector<std::array<Shared, 2>> shared(cp.nf);
+  for (int s = 0; s < kVmMaxLoads; ++s) {
+    if (cp.fam[s] < 0 || cp.dx[s] == 0 || cp.dz[s] < zl(cp.fam[s])) continue;
+    Shared& e = shared[cp.fam[s]][cp.dx[s] > 0];
+    e.ylo = std::min(e.ylo, cp.dy[s]), e.yhi = std::max(e.yhi, cp.dy[s]);
+    e.zlo = std::min(e.zlo, cp.dz[s]), e.zhi = std::max(e.zhi, cp.dz[s]);
+    e.on = e.ylo < e.yhi || e.zlo < e.zhi;
+  }
+  auto shared_reg = [](int f, int right, int j, int k) {
+    return "X" + std::to_string(f) + "_" + std::to_string(right) + "_" + std::to_string(j) + "_" + std::to_string(k);
+  };
+  // forms family f's shared neighbours of one side from plane slot k
+  auto form_shared = [&](const std::string& ind, int f, int right, int k) {
+    const Shared& e = shared[f][right];
+    o << ind << "{\n";
+    for (int j = e.ylo - cp.ylo[f]; j < RY + e.yhi - cp.ylo[f]; ++j) {
+      const std::string n = std::to_string(j);
+      o << ind << "  const double D" << n << "_ = __builtin_amdgcn_mov_dpp(" << ring(f, j, k, right ? 0 : PW - 1)
+        << ", " << (right ? "0x130" : "0x138") << ", 0xf, 0xf, true);\n";
+      o << ind << "  const double E" << n << "_ = rdlane_(" << edge_reg(f, k) << ", "
+        << (right ? 32 : 0) + j + cp.ylo[f] - ef[f].ey << ");\n";
+      o << ind << "  " << shared_reg(f, right, j, k) << " = lane_ == " << (right ? 63 : 0) << " ? E" << n << "_ : D" << n
+        << "_;\n";
+    }
+    o << ind << "}\n";
+  };
   for (int f = 0; f < cp.nf; ++f) {
     const int rows = RY + cp.yhi[f] - cp.ylo[f], ns = nslots(f);
+    for (int right = 0; right < 2; ++right)
+      for (int j = 0; shared[f][right].on && j < rows; ++j)
+        for (int k = 0; k < ns; ++k) o << "  double " << shared_reg(f, right, j, k) << " = 0.0;\n";
     for (int j = 0; j < rows; ++j)
       for (int k = 0; k < ns; ++k)
         for (int h = 0; h < PW; ++h) o << "  double " << ring(f, j, k, h) << " = 0.0;\n";
@@ -737,6 +792,10 @@ std::string jit_column_source(const VmProgram& P, const SlotUse& u, const Column
       for (int k = 0; k < ns; ++k) o << "  double " << edge_reg(f, k) << " = 0.0;\n";
     for (int k = 0; k + 1 < ns; ++k) load_plane("  ", f, k, "zs + " + std::to_string(zl(f) + k));
   }
+  for (int f = 0; f < cp.nf; ++f)
+    for (int right = 0; right < 2; ++right)
+      for (int dz = shared[f][right].zlo; shared[f][right].on && dz < shared[f][right].zhi; ++dz)
+        form_shared("  ", f, right, dz - zl(f));
   // Cells: the program as a tree, with the subtrees of shift_plan taken from the
   // row above or the plane below instead of recomputed.  Carries are written
   // after the whole cell, so a subtree taken from the previous plane always reads
@@ -818,6 +877,10 @@ std::string jit_column_source(const VmProgram& P, const SlotUse& u, const Column
         o << ind << "const double L0_" << s << " = " << val(1 - h) << ";\n";
         continue;
       }
+      if (shared[f][cp.dx[s] > 0].on && zshift == 0) {
+        o << ind << "const double L0_" << s << " = " << shared_reg(f, cp.dx[s] > 0, j, k) << ";\n";
+        continue;
+      }
       // the exchange and the edge lane's read are taken by every lane, outside
       // any branch: a lane read inside the select would run with only the edge
       // lane active, and a value the compiler keeps elsewhere (a spill) would be
@@ -838,6 +901,9 @@ std::string jit_column_source(const VmProgram& P, const SlotUse& u, const Column
     auto slot = [&](int f, int k) { return (k + u) % nslots(f); };
     for (int f = 0; f < cp.nf; ++f)
       load_plane(in, f, slot(f, nslots(f) - 1), "zq + " + std::to_string(zl(f) + nslots(f) - 1));
+    for (int f = 0; f < cp.nf; ++f)
+      for (int right = 0; right < 2; ++right)
+        if (shared[f][right].on) form_shared(in, f, right, slot(f, shared[f][right].zhi - zl(f)));
     for (size_t c = 0; c < sp.cdir.size(); ++c)
       if (sp.cdir[c] == 1)
         for (int r = 0; r + 1 < RY; ++r)
@@ -938,6 +1004,9 @@ std::string jit_column_source(const VmProgram& P, const SlotUse& u, const Column
       for (int j = 0; j < rows; ++j)
         for (int h = 0; h < PW; ++h) o << "    " << ring(f, j, k, h) << " = " << ring(f, j, k + 1, h) << ";\n";
       if (has_edge(f)) o << "    " << edge_reg(f, k) << " = " << edge_reg(f, k + 1) << ";\n";
+      for (int right = 0; right < 2; ++right)
+        for (int j = 0; shared[f][right].on && j < rows; ++j)
+          o << "    " << shared_reg(f, right, j, k) << " = " << shared_reg(f, right, j, k + 1) << ";\n";
     }
   }
   o << "  }\n}\n";
