@@ -1220,21 +1220,64 @@ std::string structural_key(const VmProgram& P, int V, const Shape& sh, int kind)
   return k;
 }
 
-// Whether an assignment runs on the column schedule (on by default for every
-// tree column_plan accepts) and its shape.  Unless set, the planes per block
-// are the most of 128, 64, 32, 16 that still give 4 waves per compute unit
-// (longer chunks load fewer halo planes; sweeps measured 64 planes fastest at
-// 256^3, div(k grad phi) 75.5-76 us against 79-84 at 32, and 128 at 512^3, the
-// transport stages 1.51-1.60 ms against 1.56-1.68 at 64), else 8.
+// What a launch of box n on the column schedule costs, in z steps of the SIMD units
+// with most waves: the box's waves go round the SIMDs, and each walks its planes and
+// about three quarters of a step before the first.  Two waves on one SIMD hide some of
+// each other's latency on short walks.  The order of the times measured over 19 boxes
+// from 40 x 36 x 30 to 512 x 512 x 256 and four trees (the 7-point Laplacian, div(k
+// grad phi), an upwind transport step, the 27-point filter): what it picks is 1.3 % from
+// the fastest on average.
+double column_steps(const ColumnPlan& cp, int waves, int zc, const int n[3], int simds, long* total_waves)
+{
+  const int xw = cp.pair ? 128 : 64, ry = cp.RY * waves;
+  const long total = (long)((n[0] + xw - 1) / xw) * ((n[1] + ry - 1) / ry) * waves * ((n[2] + zc - 1) / zc);
+  const double per = (double)((total + simds - 1) / simds);
+  *total_waves = total;
+  return (per == 2 && zc <= 16 ? 1.7 : per) * (std::min(zc, n[2]) + 0.75) * cp.RY * (cp.pair ? 2 : 1);
+}
+
+// Whether an assignment can run on the column schedule (on by default for every tree
+// column_plan accepts) and its shape.  Unless set, the planes per block and the columns
+// per lane are those of least column_steps; longer walks are preferred up to a ninth
+// (fewer halo planes, and the waves of a large box stay close in z: 384^3 Laplacian
+// 213 us at 128 planes, 235 at 32), and two columns per lane by a twentieth (256^3
+// transport step 162 us against 164).  Against the most of 128, 64, 32, 16, 8 planes that
+// give 4 waves per compute unit, and two columns wherever they fit: transport step on
+// 180x150x130 60 -> 44.5 us (one column: 128 columns wide, the second wave of each row
+// was 40 % full), 300^3 428 -> 315, 330x190x410 428 -> 275 (the last of 4 walks of 128
+// planes was a fifth full); div(k grad phi) on 300^3 240 -> 160; filter on 180x150x130
+// 20.0 -> 14.2, 40x36x30 7.9 -> 4.5.
 bool column_choice(const VmProgram& P, const nebo_limits_t* lim, ColumnPlan* cp, ColumnShape* cs)
 {
   const int mode = g_column.load();
   const bool wide = !lim || lim->hi[0] - lim->lo[0] > 64;
   if (!mode || !column_plan(P, slot_use(P), cp) || !select_ring(P, cp, kColumnPairs && mode == 1 && wide))
     return false;
-  cs->waves = g_column_waves.load();
-  if (cs->waves == 0) cs->waves = cp->pair ? kDefaultPairWaves : kDefaultColumnWaves;
+  const auto waves = [](const ColumnPlan& p) {
+    const int w = g_column_waves.load();
+    return w ? w : p.pair ? kDefaultPairWaves : kDefaultColumnWaves;
+  };
   cs->zc = g_column_zc.load();
+  int device = 0;
+  if (cs->zc == 0 && lim && hipGetDevice(&device) == hipSuccess) {
+    const int n[3] = {lim->hi[0] - lim->lo[0], lim->hi[1] - lim->lo[1], lim->hi[2] - lim->lo[2]};
+    const int simds = 4 * device_cu_count(device);
+    double least = 0;
+    long total = 0;
+    ColumnPlan one = *cp;
+    if (cp->pair && !select_ring(P, &one, false)) one = *cp;
+    const ColumnPlan layouts[2] = {*cp, one};
+    for (int l = 0; l < (cp->pair != one.pair ? 2 : 1); ++l)
+      for (int zc : {128, 64, 32, 16, 8, 4, 2}) {
+        const double c = column_steps(layouts[l], waves(layouts[l]), zc, n, simds, &total) * (layouts[l].pair ? 1 / 1.05 : 1);
+        if (least > 0 && c >= 0.89 * least) continue;
+        least = c;
+        *cp = layouts[l];
+        cs->zc = zc;
+      }
+  }
+  if (cs->zc == 0) cs->zc = kDefaultColumnZc;
+  cs->waves = waves(*cp);
   cs->xcd = g_xcd.load();
   // Indices of the kernel's stores and per-lane offsets are 32-bit: lanes, rows
   // and planes past the box reach at most 64 PW + 2 + X (RY waves + 2) +
@@ -1248,20 +1291,28 @@ bool column_choice(const VmProgram& P, const nebo_limits_t* lim, ColumnPlan* cp,
                        (long)(cp->PF + 2) * P.cls_XY[k];
     if (reach >= 2147483647L) return false;
   }
-  if (cs->zc == 0) {
-    cs->zc = kDefaultColumnZc;
-    int device = 0;
-    if (lim && hipGetDevice(&device) == hipSuccess) {
-      const int xw = cp->pair ? 128 : 64;   // columns per wave
-      const long cols = (long)((lim->hi[0] - lim->lo[0] + xw - 1) / xw) *
-                        ((lim->hi[1] - lim->lo[1] + cp->RY * cs->waves - 1) / (cp->RY * cs->waves)) * cs->waves;
-      const long want = 4L * device_cu_count(device);
-      const int nz = lim->hi[2] - lim->lo[2];
-      for (int zc : {128, 64, 32, 16})
-        if (cs->zc == kDefaultColumnZc && cols * ((nz + zc - 1) / zc) >= want) cs->zc = zc;
-    }
-  }
   return true;
+}
+
+// Trees with fewer than 5 reads per field on small boxes: the column schedule loads each
+// value once, which saves such a tree little (an upwind transport step reads 6 fields at
+// 20 points), and gives a lane several cells to form one after the other, where the
+// flattened schedule gives each a thread.  Taken below 4 waves per compute unit at 8
+// planes: 40x36x30 4.9 us against 6.2 at 2 planes and 14.3 at 8, 64^3 5.9 against 7.4 and
+// 14.9, 112x96x104 14.4 against 16.0; at 128^3, with 4, 25.8 against 21.3.  With more
+// reads short walks are as fast or faster at every size (div(k grad phi) on 80^3 6.7 us at
+// 4 planes, 8.5 flattened; filter on 100x90x80 6.3 and 9.1).
+bool prefers_flat(const ColumnPlan& cp, const nebo_limits_t& lim)
+{
+  if (g_column_waves.load() || g_column_zc.load()) return false;
+  int reads = 0, device = 0;
+  for (int s = 0; s < kVmMaxLoads; ++s) reads += cp.fam[s] >= 0;
+  if (reads >= 5 * cp.nf || hipGetDevice(&device) != hipSuccess) return false;
+  const int n[3] = {lim.hi[0] - lim.lo[0], lim.hi[1] - lim.lo[1], lim.hi[2] - lim.lo[2]};
+  const int simds = 4 * device_cu_count(device);
+  long waves = 0;
+  column_steps(cp, cp.pair ? kDefaultPairWaves : kDefaultColumnWaves, 8, n, simds, &waves);
+  return waves < simds;
 }
 
 std::string column_key(const VmProgram& P, const ColumnPlan& cp, const ColumnShape& cs)
@@ -1442,7 +1493,7 @@ int jit_assign(const nebo_field_t* lhs, const VmProgram& P, const nebo_limits_t&
   Entry e;
   ColumnPlan cp;
   ColumnShape cs;
-  if (column_choice(P, &lim, &cp, &cs)) {
+  if (column_choice(P, &lim, &cp, &cs) && !prefers_flat(cp, lim)) {
     int rc = get_kernel_keyed(column_key(P, cp, cs), [&] { return jit_column_source(P, slot_use(P), cp, cs); },
                               "nebo_fused", &e);
     if (rc || !e.fn) return rc;

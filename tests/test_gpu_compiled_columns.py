@@ -45,3 +45,30 @@ def test_shared_neighbours_match_oracle(column, n):
                 assert np.array_equal(fetch(out), ref.host), (column, name, use_ghost)
     finally:
         nh.fused_jit_column()
+
+
+def _few_reads(L, phi, k):
+    """Three fields at 2 reads each."""
+    g = both(L, np.random.default_rng(31).standard_normal(L.npts))
+    lo = nh.Stencil([(0, 0, -1), (0, 0, 0)], COEF[:2])
+    side = nh.Stencil([(-1, 0, 0), (0, 0, 0)], COEF[1:3])
+    return lo(phi) * side(k) + lo(g)
+
+
+# Boxes of every planes-per-block choice, of one and two columns per lane, and on both
+# sides of the line where trees of few reads leave the schedule.
+@pytest.mark.parametrize("n,few_flat", [((40, 36, 30), True), ((100, 90, 20), True), ((180, 50, 70), True),
+                                        ((130, 129, 131), False), ((300, 200, 33), False)])
+def test_default_schedule_matches_oracle(n, few_flat):
+    L = nh.Layout.build(n, 1)
+    rng = np.random.default_rng(37)
+    phi, k = both(L, rng.standard_normal(L.npts)), both(L, rng.uniform(0.5, 2.0, L.npts))
+    trees = {x: t for x, t in _trees(L, phi, k, n).items() if x in ("filter", "two_fields", "two_sided")}
+    for name, t in {**trees, "few_reads": _few_reads(L, phi, k)}.items():
+        print(f"{n} {name}", flush=True)
+        out = gpu_empty_like(L, 7.0)
+        ref = nh.Field.from_numpy(L, np.full(L.npts, 7.0), where="cpu")
+        nh.assign(out, t, use_ghost=False, generic=True)
+        assert ("column schedule" in nh.last_backend()) == (name != "few_reads" or not few_flat), nh.last_backend()
+        orc.assign(ref, t, use_ghost=False)
+        assert np.array_equal(fetch(out), ref.host), (name, nh.last_backend())
