@@ -144,7 +144,7 @@ __device__ __forceinline__ double lane_gather(double v, int src)
   return __hiloint2double(hi, lo);
 }
 
-template <int RY, int PF>
+template <int RY, int PF, int SP>
 __global__ __launch_bounds__(256) void batch_column_kernel(const DevPatch* __restrict__ P,
                                                            const int4* __restrict__ items, int n_items, int zc,
                                                            Coef6 c, double s, int swap)
@@ -223,7 +223,7 @@ __global__ __launch_bounds__(256) void batch_column_kernel(const DevPatch* __res
       const double Ly = (pym * c.gy0 + pc * c.gy1) * c.dy0 + (pc * c.gy0 + pyp * c.gy1) * c.dy1;
       const double Lz = gz[j] * c.dz0 + gz_hi * c.dz1;
       gz[j] = gz_hi;
-      if (active && yb + j < p.ny) store_nt_at(ro, row[j + 1], pc + s * ((Lx + Ly) + Lz));
+      if (active && yb + j < p.ny) store_at<SP>(ro, row[j + 1], pc + s * ((Lx + Ly) + Lz));
     }
     // the slot's next plane is read by step z + NS - 1 at the earliest: past the
     // item's last plane (z1) no step reads it (z is uniform over the wave)
@@ -281,6 +281,7 @@ struct nebo_batch {
   std::vector<int> patch_first;   // first item of each patch (items are grouped by patch)
   int blocks = 0;
   long max_plane = 0;   // largest (nx+2)*(ny+2) of the patches
+  long bytes = 0;       // of both blocks of every patch
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
 };
@@ -368,18 +369,31 @@ int check_tile(const int32_t* t)
 // for 16-plane items 3 planes ahead; 4-plane items took 0.151 ms 3 planes ahead and
 // 0.121-0.155 ms 5-9 ahead (whose first loads repeat the item's last plane).
 using ColumnKernel = void (*)(const DevPatch*, const int4*, int, int, Coef6, double, int);
+template <int SP>
 ColumnKernel column_kernel(int ry, int zc)
 {
-  if (zc <= 4) return ry == 1 ? batch_column_kernel<1, 4> : ry == 2 ? batch_column_kernel<2, 4> : batch_column_kernel<4, 4>;
-  if (zc <= 8) return ry == 1 ? batch_column_kernel<1, 8> : ry == 2 ? batch_column_kernel<2, 8> : batch_column_kernel<4, 8>;
-  return ry == 1 ? batch_column_kernel<1, 3> : ry == 2 ? batch_column_kernel<2, 3> : batch_column_kernel<4, 2>;
+  if (zc <= 4)
+    return ry == 1 ? batch_column_kernel<1, 4, SP> : ry == 2 ? batch_column_kernel<2, 4, SP> : batch_column_kernel<4, 4, SP>;
+  if (zc <= 8)
+    return ry == 1 ? batch_column_kernel<1, 8, SP> : ry == 2 ? batch_column_kernel<2, 8, SP> : batch_column_kernel<4, 8, SP>;
+  return ry == 1 ? batch_column_kernel<1, 3, SP> : ry == 2 ? batch_column_kernel<2, 3, SP> : batch_column_kernel<4, 2, SP>;
 }
+
+// Stores are written back where both blocks of every patch fit the 256 MB memory-side
+// cache, which the next step then reads them from, and go past it where they do not, so
+// that they leave it to the reads.  Patches of 16-64^3 stepped back and forth (and one
+// direction on three sets in turn), written back against past it: 69 MB in all 14.9 us
+// against 16.9 (14.9 and 16.9), 150 MB 26.4 and 33.5 (44.5 and 51.5), 211 MB 34.2 and
+// 46.4 (59.6 and 70.8), 243 MB 39 and 53 (67 and 73); 280 MB 59.3 and 61.5 (77.5 and
+// 73.2), 580 MB 154 and 138 (154 and 140).
+constexpr long kWriteBackBytes = 250000000;
 
 int launch_items(nebo_batch* b, int first, int count, int grid, int swap, hipStream_t s)
 {
   if (count <= 0) return NEBO_OK;
   if (b->tile[0] == 0) {
-    const ColumnKernel fn = column_kernel(b->tile[1], b->tile[2]);
+    const ColumnKernel fn = b->bytes <= kWriteBackBytes ? column_kernel<0>(b->tile[1], b->tile[2])
+                                                        : column_kernel<2>(b->tile[1], b->tile[2]);
     hipLaunchKernelGGL(fn, dim3((count + 3) / 4), dim3(256), 0, s, b->d_patches, b->d_items + first, count,
                        b->tile[2], coef6(b->coefs), b->s, swap);
   } else if (b->tile[1] == 0) {
@@ -419,11 +433,15 @@ extern "C" int nebo_batch_create(const nebo_patch_t* patches, int32_t n, const n
   long max_plane = 0;
   for (int i = 0; i < n; ++i)
     max_plane = std::max(max_plane, (long)(patches[i].n[0] + 2) * (patches[i].n[1] + 2));
+  long bytes = 0;
+  for (int i = 0; i < n; ++i)
+    bytes += 16L * (patches[i].n[0] + 2) * (patches[i].n[1] + 2) * (patches[i].n[2] + 2);
   // the column schedule addresses a plane with 32-bit byte offsets
   if (tile && tile[0] == 0 && max_plane * 8 >= (1L << 31))
     return set_error(NEBO_ERR_TOO_LARGE, ctx, "a column tile needs every patch plane below 2^31 bytes");
   nebo_batch* b = new nebo_batch;
   b->max_plane = max_plane;
+  b->bytes = bytes;
   b->patches.assign(patches, patches + n);
   b->coefs = *c;
   b->s = s;
