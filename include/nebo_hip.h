@@ -263,7 +263,9 @@ int nebo_set_fused_jit(int enable);
  * blocks so that neighbouring tiles run on one XCD (one L2).  0 keeps the
  * default of block_threads, max_cells and load_budget, -1 that of tile_x and
  * xcd_remap.  Defaults: 512 threads, flattened plane, 4 cells, 48 reads, XCD
- * renumbering on.  Kernels compiled for another shape stay cached. */
+ * renumbering on; while block_threads, tile_x and max_cells are all at their
+ * defaults, an assignment takes 256 threads and 1, 2 or 4 cells by its box and
+ * its reads.  Kernels compiled for another shape stay cached. */
 int nebo_fused_jit_tune(int32_t block_threads, int32_t tile_x, int32_t max_cells,
                         int32_t load_budget, int32_t xcd_remap);
 /* Column schedule of the compiled assignment kernels.  It applies to a tree
@@ -278,8 +280,11 @@ int nebo_fused_jit_tune(int32_t block_threads, int32_t tile_x, int32_t max_cells
  * trees keep the shape of nebo_fused_jit_tune.  mode 1 uses it where it
  * applies (the default), 2 the same with one column per lane, 0 never; waves
  * per block (stacked in y) in [1, 16], 0 (the default) for 4 with two columns
- * per lane and 1 with one; zchunk in [1, 4096], 0 (the default) for the most of
- * 128, 64, 32 or 16 planes that still gives 4 waves per compute unit, else 8.
+ * per lane and 1 with one; zchunk in [1, 4096], 0 (the default) for the power of
+ * two from 2 to 128, and one or two columns, whose rounds of waves walk the fewest
+ * planes on the box.  While waves and zchunk are 0, trees with fewer than 5 reads
+ * per field keep the shape of nebo_fused_jit_tune on boxes of less than 4 waves of
+ * 8 planes per compute unit.
  * Results are the same bits either way. */
 int nebo_fused_jit_column(int32_t mode, int32_t waves, int32_t zchunk);
 int nebo_fused_jit_stats(int32_t* compiled, int32_t* cache_hits, int32_t* failures);

@@ -77,16 +77,13 @@ static_assert(kVmMaxLoads == 40 && kVmMaxMasks == 6 && kVmMaxConsts == 48 && kVm
 constexpr int kReduceBlock = 256;   // threads per block of the reduction kernels
 
 // Launch shape of the assignment kernels and the cells-per-thread rule (see
-// choose_cells); 0 in nebo_fused_jit_tune restores these defaults.
-// Defaults from a sweep at 256^3 (pointwise, cond, Laplacian and div(k grad phi)
-// trees): 512-thread blocks over the flattened plane, XCD renumbering on, up to
-// 4 cells per thread within 48 distinct reads.  Larger blocks let a block's rows
-// share their y-neighbour rows in L1; 2-D tiles and 8 cells per thread measured
-// slower.
+// choose_cells); 0 in nebo_fused_jit_tune restores these defaults, and the shape an
+// assignment then takes is flat_shape's.
 constexpr int kDefaultBlock = 512, kDefaultTileX = 0, kDefaultMaxCells = 4, kDefaultLoadBudget = 48,
               kDefaultXcd = 1;
 std::atomic<int> g_block{kDefaultBlock}, g_tile_x{kDefaultTileX}, g_max_cells{kDefaultMaxCells},
     g_load_budget{kDefaultLoadBudget}, g_xcd{kDefaultXcd};
+std::atomic<bool> g_shape_set{false};   // block_threads, tile_x or max_cells chosen by the caller
 constexpr int kXcds = 8;   // MI355X: 8 accelerator complex dies, each with its own L2
 
 // Launch shape of an assignment kernel: threads per block; tile_x == 0 lays the
@@ -1394,6 +1391,29 @@ int choose_cells(const VmProgram& P)
   return V;
 }
 
+// Shape and cells per thread of a flattened assignment, unless the caller set them:
+// 256 threads, and cells for about 4 values a thread reads at once (2 cells of two
+// fields, 4 of one), fewer where that leaves a CU less than half its waves (4 cells: all
+// of them).  Blocks of 512 threads with 4 cells, taken at all sizes before, gave small
+// boxes a few long waves: phi/2 + k on 48x40x36 2.9 -> 2.4 us, 80^3 3.9 -> 3.2, 128^3
+// 9.7 -> 9.4, 256x256x160 50 -> 47; a masked cond 2.8 -> 2.3, 3.4 -> 3.2, 7.6 -> 7.4
+// and (4 cells) 29.4; an upwind transport step (512 threads, 2 cells) 4.6 -> 3.4 on
+// 48x40x36, 8.7 -> 7.7 on 80^3, 14.1 -> 12.5 on 112x96x104.
+int flat_shape(const VmProgram& P, const nebo_limits_t& lim, Shape* sh)
+{
+  const int most = choose_cells(P);
+  int device = 0;
+  *sh = current_shape();
+  if (g_shape_set.load() || hipGetDevice(&device) != hipSuccess) return most;
+  sh->block = 256;
+  SlotUse u = slot_use(P);
+  for (int m = 0; m < kVmMaxMasks; ++m) u.mused[m] = false;   // bits: next to no bytes
+  const double waves = (double)(lim.hi[0] - lim.lo[0]) * (lim.hi[1] - lim.lo[1]) * (lim.hi[2] - lim.lo[2]) / 64 /
+                       device_cu_count(device);
+  const int V = reads_per_thread(u, 4) <= 4 && waves >= 4 * 32 ? 4 : waves >= 2 * 16 ? 2 : 1;
+  return std::min(V, most);
+}
+
 // Cells per thread of a reduction: the assignment's count, doubled (up to 16)
 // while a thread issues fewer than 8 loads per item, the reads stay within the
 // load budget and the box still gives every thread of a full grid (max_blocks
@@ -1488,8 +1508,8 @@ int jit_assign(const nebo_field_t* lhs, const VmProgram& P, const nebo_limits_t&
 {
   *done = false;
   if (!jit_enabled()) return NEBO_OK;
-  const int V = choose_cells(P);
-  const Shape sh = current_shape();
+  Shape sh;
+  const int V = flat_shape(P, lim, &sh);
   Entry e;
   ColumnPlan cp;
   ColumnShape cs;
@@ -1611,6 +1631,7 @@ extern "C" int nebo_fused_jit_tune(int32_t block_threads, int32_t tile_x, int32_
     return nebo::set_error(NEBO_ERR_INVALID, ctx, "max_cells: a power of two in [1, 16]");
   if (l < 1 || l > 256) return nebo::set_error(NEBO_ERR_INVALID, ctx, "load_budget: in [1, 256]");
   if (x != 0 && x != 1) return nebo::set_error(NEBO_ERR_INVALID, ctx, "xcd_remap: 0 or 1");
+  nebo::g_shape_set.store(block_threads != 0 || tile_x > 0 || max_cells != 0);
   nebo::g_block.store(b);
   nebo::g_tile_x.store(tx);
   nebo::g_max_cells.store(m);

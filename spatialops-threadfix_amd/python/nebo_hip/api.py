@@ -139,15 +139,17 @@ def fused_jit_column(enable=True, waves=0, zchunk=0):
     allows), each lane 1-4 rows and `zchunk` planes, and each plane of each field
     is loaded once.  enable: True/1 on, 2 on with one column per lane, False/0
     off.  0 keeps the defaults (1 wave per block; planes per block from the box
-    size: 128, 64, 32, 16 or 8)."""
+    size: a power of two from 2 to 128; trees of few reads leave the schedule on
+    small boxes)."""
     mode = 2 if enable == 2 else int(bool(enable))
     _abi.call("nebo_fused_jit_column", mode, int(waves), int(zchunk))
 
 
 def fused_jit_tune(block_threads=0, tile_x=-1, max_cells=0, load_budget=0, xcd_remap=-1):
     """Launch shape of the compiled assignment kernels; the defaults restore the
-    library's own (512 threads over the flattened plane, up to 4 z cells per
-    thread within 48 distinct reads, XCD renumbering on)."""
+    library's own (256 threads over the flattened plane and 1, 2 or 4 z cells per
+    thread by the box and the reads, within 48 distinct reads, XCD renumbering on;
+    512 threads where only some are set)."""
     _abi.call("nebo_fused_jit_tune", int(block_threads), int(tile_x), int(max_cells), int(load_budget),
               int(xcd_remap))
 

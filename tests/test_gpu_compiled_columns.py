@@ -72,3 +72,23 @@ def test_default_schedule_matches_oracle(n, few_flat):
         assert ("column schedule" in nh.last_backend()) == (name != "few_reads" or not few_flat), nh.last_backend()
         orc.assign(ref, t, use_ghost=False)
         assert np.array_equal(fetch(out), ref.host), (name, nh.last_backend())
+
+
+# Boxes of 1, 2 and 4 cells per thread, with planes below and past one block and z
+# extents that cut the last cells.
+@pytest.mark.parametrize("n,masked_cells", [((5, 3, 2), 1), ((33, 31, 30), 1), ((129, 90, 50), 2),
+                                            ((160, 131, 111), 4)])
+def test_flattened_shapes_match_oracle(n, masked_cells):
+    L = nh.Layout.build(n, 1)
+    rng = np.random.default_rng(41)
+    phi, k = both(L, rng.standard_normal(L.npts)), both(L, rng.uniform(0.5, 2.0, L.npts))
+    m = nh.Mask(L, [(x, y, n[2] - 1) for x in range(n[0]) for y in range(0, n[1], 2)]).add_consumer(0)
+    for name, t in {"masked": nh.cond(m, 0.25)(phi), "two": 0.5 * phi + k}.items():
+        for use_ghost in (True, False):
+            out = gpu_empty_like(L, 7.0)
+            ref = nh.Field.from_numpy(L, np.full(L.npts, 7.0), where="cpu")
+            nh.assign(out, t, use_ghost=use_ghost, generic=True)
+            cells = masked_cells if name == "masked" else min(masked_cells, 2)
+            assert f"{cells} z cells per thread (256-thread blocks)" in nh.last_backend(), nh.last_backend()
+            orc.assign(ref, t, use_ghost=use_ghost)
+            assert np.array_equal(fetch(out), ref.host), (name, use_ghost, nh.last_backend())
