@@ -354,8 +354,7 @@ extern "C" int nebo_diffusion_forward(const nebo_field_t* phiT, const nebo_field
   double* tmp = nullptr;
   if ((rc = scratch_alloc((void**)&tmp, 2 * bytes, s, kCtx))) return rc;
   nebo_field_t ck0 = with_values(phi0, ckpt);
-  rc = check_hip(hipMemcpyAsync(ckpt, phi0->values, bytes, hipMemcpyDeviceToDevice, s), kCtx);
-  if (!rc) rc = fill_ghosts_periodic(&ck0, stream);
+  rc = copy_periodic(&ck0, phi0->values, nullptr, stream);
   double* cur = ckpt;
   for (int st = 0; st < n_steps && !rc; ++st) {
     double* dst;
@@ -387,15 +386,15 @@ extern "C" int nebo_diffusion_backward(const nebo_field_t* lam0, double* gk, con
       (rc = check_periodic_field(k, lamT)))
     return rc;
   if (lam0->values == lamT->values) return set_error(NEBO_ERR_INVALID, kCtx, "lam0 must not alias lamT");
-  hipStream_t s = (hipStream_t)stream;
-  const size_t np = field_npts(lamT), bytes = np * sizeof(double);
-  // lam ping-pongs between work slot `every` and lam0
-  double* lbuf[2] = {work + (size_t)every * np, static_cast<double*>(lam0->values)};
+  const size_t np = field_npts(lamT);
+  // lam goes back and forth between work slot `every` and lam0, so that the last step
+  // ends in lam0
+  double* end = static_cast<double*>(lam0->values);
+  double* slot = work + (size_t)every * np;
+  double* lbuf[2] = {n_steps % 2 ? slot : end, n_steps % 2 ? end : slot};
   int cur = 0;
   nebo_field_t L0 = with_values(lamT, lbuf[0]);
-  rc = check_hip(hipMemcpyAsync(lbuf[0], lamT->values, bytes, hipMemcpyDeviceToDevice, s), kCtx);
-  if (!rc) rc = fill_ghosts_periodic(&L0, stream);
-  if (!rc) rc = check_hip(hipMemsetAsync(gk, 0, field_npts(k) * sizeof(double), s), kCtx);
+  rc = copy_periodic(&L0, lamT->values, gk, stream);
   const int nseg = n_steps / every;
   for (int seg = nseg - 1; seg >= 0 && !rc; --seg) {
     // recompute states every*seg ... every*seg + every - 1 (state 0 of the segment is the checkpoint)
@@ -415,7 +414,5 @@ extern "C" int nebo_diffusion_backward(const nebo_field_t* lam0, double* gk, con
       cur = 1 - cur;
     }
   }
-  if (!rc && lbuf[cur] != lam0->values)
-    rc = check_hip(hipMemcpyAsync(lam0->values, lbuf[cur], bytes, hipMemcpyDeviceToDevice, s), kCtx);
   return rc;
 }

@@ -234,6 +234,9 @@ int launch_diffusion_euler(const nebo_field_t* out, const nebo_field_t* k, const
 int fill_thin_ghosts(const nebo_field_t* f, void* stream);
 // Periodic copy-fill of every allocated ghost layer of f.
 int fill_ghosts_periodic(const nebo_field_t* f, void* stream);
+// out = the block `in` with every ghost layer filled periodically; zero, if not null, a
+// block of the same size to clear.
+int copy_periodic(const nebo_field_t* out, const void* in, double* zero, void* stream);
 
 // Periodic operands (diffusion and transport chains): f shares ref's memory
 // window and device, has exactly one ghost layer per face (valid) and fewer than

@@ -1059,6 +1059,52 @@ __global__ __launch_bounds__(256) void fill_periodic_kernel(double* __restrict__
   v[dst[0] + (long)A.X * (dst[1] + (long)A.Y * dst[2])] = v[src[0] + (long)A.X * (src[1] + (long)A.Y * src[2])];
 }
 
+// out = in with every ghost cell replaced by the interior cell it is the image of, and
+// zero (if any) cleared: where a trajectory starts, in one pass over the block (128^3: a
+// copy, a fill and a clearing of 17 MB took 6.2 + 4.6 + 5.3 us, this 10).  out may be in.
+__global__ __launch_bounds__(256) void copy_periodic_kernel(double* out, const double* in, double* zero, FillArgs A,
+                                                            long npts)
+{
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= npts) return;
+  const int u = (int)(t / A.X);
+  const int c[3] = {(int)(t - (long)u * A.X), u % A.Y, u / A.Y};
+  int src[3];
+  bool inside = true;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const int w = c[a] - A.o[a];
+    inside = inside && w >= 0 && w < A.e[a];
+    const int rel = w - A.gm[a];   // at most n cells from the interior on either side
+    src[a] = c[a] + (rel < 0 ? A.n[a] : rel >= A.n[a] ? -A.n[a] : 0);
+  }
+  out[t] = in[inside ? src[0] + (long)A.X * (src[1] + (long)A.Y * src[2]) : t];
+  if (zero) zero[t] = 0.0;
+}
+
+// The slabs of f's ghost layers; NEBO_ERR_GHOST where an axis has too few cells.
+int fill_args(const nebo_field_t* f, FillArgs* A)
+{
+  A->X = f->glob[0];
+  A->Y = f->glob[1];
+  A->total = 0;
+  for (int d = 0; d < 3; ++d) {
+    A->o[d] = f->offset[d];
+    A->e[d] = f->extent[d];
+    A->gm[d] = f->ghost_minus[d];
+    A->gp[d] = f->ghost_plus[d];
+    A->n[d] = f->extent[d] - f->ghost_minus[d] - f->ghost_plus[d];
+    if ((A->gm[d] > 0 || A->gp[d] > 0) && (A->n[d] < A->gm[d] || A->n[d] < A->gp[d]))
+      return set_error(NEBO_ERR_GHOST, "Nebo Ghost Fill", "fewer interior cells than ghost layers on a periodic axis");
+    A->first[d] = A->total;
+    long slab = A->gm[d] + A->gp[d];
+    for (int a = 0; a < 3; ++a)
+      if (a != d) slab *= f->extent[a];
+    A->total += slab;
+  }
+  return NEBO_OK;
+}
+
 }  // namespace
 
 int launch_divkgrad(const nebo_field_t* r, const nebo_field_t* k, const nebo_field_t* phi,
@@ -1094,35 +1140,25 @@ int launch_lapl_euler(const nebo_field_t* out, const nebo_field_t* phi,
 
 int fill_ghosts_periodic(const nebo_field_t* f, void* stream)
 {
-  static const char* ctx = "Nebo Ghost Fill";
-  int n[3];
-  for (int d = 0; d < 3; ++d) {
-    n[d] = f->extent[d] - f->ghost_minus[d] - f->ghost_plus[d];
-    if ((f->ghost_minus[d] > 0 || f->ghost_plus[d] > 0) &&
-        (n[d] < f->ghost_minus[d] || n[d] < f->ghost_plus[d]))
-      return set_error(NEBO_ERR_GHOST, ctx, "fewer interior cells than ghost layers on a periodic axis");
-  }
   FillArgs A;
-  A.X = f->glob[0];
-  A.Y = f->glob[1];
-  A.total = 0;
-  for (int d = 0; d < 3; ++d) {
-    A.o[d] = f->offset[d];
-    A.e[d] = f->extent[d];
-    A.gm[d] = f->ghost_minus[d];
-    A.gp[d] = f->ghost_plus[d];
-    A.n[d] = n[d];
-    A.first[d] = A.total;
-    long slab = A.gm[d] + A.gp[d];
-    for (int a = 0; a < 3; ++a)
-      if (a != d) slab *= f->extent[a];
-    A.total += slab;
-  }
+  if (int rc = fill_args(f, &A)) return rc;
   if (A.total <= 0) return NEBO_OK;
   const int blk = 256;
   hipLaunchKernelGGL(fill_periodic_kernel, dim3((unsigned)((A.total + blk - 1) / blk)), dim3(blk), 0,
                      (hipStream_t)stream, static_cast<double*>(f->values), A);
-  return check_hip(hipGetLastError(), ctx);
+  return check_hip(hipGetLastError(), "Nebo Ghost Fill");
+}
+
+int copy_periodic(const nebo_field_t* out, const void* in, double* zero, void* stream)
+{
+  FillArgs A;
+  if (int rc = fill_args(out, &A)) return rc;
+  const long npts = (long)field_npts(out);
+  if (npts <= 0) return NEBO_OK;
+  const int blk = 256;
+  hipLaunchKernelGGL(copy_periodic_kernel, dim3((unsigned)((npts + blk - 1) / blk)), dim3(blk), 0, (hipStream_t)stream,
+                     static_cast<double*>(out->values), static_cast<const double*>(in), zero, A, npts);
+  return check_hip(hipGetLastError(), "Nebo Ghost Fill");
 }
 
 namespace {

@@ -693,7 +693,8 @@ int check_operands(const nebo_field_t* ref, const nebo_field_t* k, const nebo_fi
   return NEBO_OK;
 }
 
-// One RK3 step phi_n -> phi_next through s1, s2 (all periodic-filled).
+// One RK3 step phi_n -> phi_next through s1, s2 (all periodic-filled); next may be null,
+// when s1 and s2 are all that is wanted.
 int rk3_step(double* next, double* s1, double* s2, const double* phin, const nebo_field_t* ref,
              const Operands& o, const nebo_axis_coefs_t& c, double dt, void* stream)
 {
@@ -701,7 +702,7 @@ int rk3_step(double* next, double* s1, double* s2, const double* phin, const neb
   const nebo_field_t S1 = with_values(ref, s1), S2 = with_values(ref, s2), N = with_values(ref, next);
   int rc = launch_stage(&S1, &P, &P, o, c, dt, 1, stream);
   if (!rc) rc = launch_stage(&S2, &P, &S1, o, c, dt, 2, stream);
-  if (!rc) rc = launch_stage(&N, &P, &S2, o, c, dt, 3, stream);
+  if (!rc && next) rc = launch_stage(&N, &P, &S2, o, c, dt, 3, stream);
   return rc;
 }
 
@@ -793,8 +794,7 @@ extern "C" int nebo_transport_forward(const nebo_field_t* phiT, const nebo_field
   if ((rc = scratch_alloc((void**)&tmp, 4 * bytes, st, kCtx))) return rc;
   const Operands o{u, k};
   nebo_field_t ck0 = with_values(phi0, ckpt);
-  rc = check_hip(hipMemcpyAsync(ckpt, phi0->values, bytes, hipMemcpyDeviceToDevice, st), kCtx);
-  if (!rc) rc = fill_ghosts_periodic(&ck0, stream);
+  rc = copy_periodic(&ck0, phi0->values, nullptr, stream);
   double* cur = ckpt;
   for (int n = 0; n < n_steps && !rc; ++n) {
     double* dst;
@@ -822,8 +822,7 @@ extern "C" int nebo_transport_backward(const nebo_field_t* lam0, double* gk, con
   int rc;
   if ((rc = check_operands(lamT, k, u)) || (rc = check_periodic_operand(lam0, lamT, kCtx))) return rc;
   if (lam0->values == lamT->values) return set_error(NEBO_ERR_INVALID, kCtx, "lam0 must not alias lamT");
-  hipStream_t st = (hipStream_t)stream;
-  const size_t np = field_npts(lamT), bytes = np * sizeof(double);
+  const size_t np = field_npts(lamT);
   const Operands o{u, k};
   // work: states (phi_n, s1, s2) of one segment's steps, then lam, mu2, mu1, acc, acc2
   double* states = work;
@@ -832,35 +831,34 @@ extern "C" int nebo_transport_backward(const nebo_field_t* lam0, double* gk, con
   double* mu1 = mu2 + np;
   double* acc = mu1 + np;
   double* acc2 = acc + np;
-  double* lbuf[2] = {lamA, static_cast<double*>(lam0->values)};
+  // lam goes back and forth between work and lam0, so that the last step ends in lam0
+  double* end = static_cast<double*>(lam0->values);
+  double* lbuf[2] = {n_steps % 2 ? lamA : end, n_steps % 2 ? end : lamA};
   int cur = 0;
   nebo_field_t L0 = with_values(lamT, lbuf[0]);
-  rc = check_hip(hipMemcpyAsync(lbuf[0], lamT->values, bytes, hipMemcpyDeviceToDevice, st), kCtx);
-  if (!rc) rc = fill_ghosts_periodic(&L0, stream);
-  if (!rc) rc = check_hip(hipMemsetAsync(gk, 0, field_npts(k) * sizeof(double), st), kCtx);
+  rc = copy_periodic(&L0, lamT->values, gk, stream);
   const int nseg = n_steps / every;
   for (int seg = nseg - 1; seg >= 0 && !rc; --seg) {
-    // recompute the segment: states[t] = (phi_t, s1_t, s2_t), phi_0 = the checkpoint
-    rc = check_hip(hipMemcpyAsync(states, ckpt + (size_t)seg * np, bytes, hipMemcpyDeviceToDevice, st), kCtx);
+    // recompute the segment: states[t] = (phi_t, s1_t, s2_t), phi_0 = the checkpoint; the
+    // last step's next state is a checkpoint already, so it stops at s2
+    const double* first = ckpt + (size_t)seg * np;
+    auto state = [&](int t) { return t ? states + (size_t)3 * t * np : const_cast<double*>(first); };
     for (int t = 0; t < every && !rc; ++t) {
-      double* phit = states + (size_t)3 * t * np;
-      double* nxt = t + 1 < every ? states + (size_t)3 * (t + 1) * np : mu2;   // last next is not kept
-      rc = rk3_step(nxt, phit + np, phit + 2 * np, phit, lamT, o, *c, dt, stream);
+      double* s1 = states + (size_t)3 * t * np + np;
+      rc = rk3_step(t + 1 < every ? state(t + 1) : nullptr, s1, s1 + np, state(t), lamT, o, *c, dt, stream);
     }
     for (int t = every - 1; t >= 0 && !rc; --t) {
-      const double* phit = states + (size_t)3 * t * np;
+      const double* s1 = states + (size_t)3 * t * np + np;
       const nebo_field_t Lin = with_values(lamT, lbuf[cur]), Lout = with_values(lamT, lbuf[1 - cur]);
       const nebo_field_t M2 = with_values(lamT, mu2), M1 = with_values(lamT, mu1);
-      const nebo_field_t Pn = with_values(lamT, const_cast<double*>(phit));
-      const nebo_field_t S1 = with_values(lamT, const_cast<double*>(phit + np));
-      const nebo_field_t S2 = with_values(lamT, const_cast<double*>(phit + 2 * np));
+      const nebo_field_t Pn = with_values(lamT, state(t));
+      const nebo_field_t S1 = with_values(lamT, const_cast<double*>(s1));
+      const nebo_field_t S2 = with_values(lamT, const_cast<double*>(s1 + np));
       rc = launch_adjoint(&M2, acc, gk, &Lin, nullptr, &S2, o, *c, dt, 3, stream);
       if (!rc) rc = launch_adjoint(&M1, acc2, gk, &M2, acc, &S1, o, *c, dt, 2, stream);
       if (!rc) rc = launch_adjoint(&Lout, nullptr, gk, &M1, acc2, &Pn, o, *c, dt, 1, stream);
       cur = 1 - cur;
     }
   }
-  if (!rc && lbuf[cur] != lam0->values)
-    rc = check_hip(hipMemcpyAsync(lam0->values, lbuf[cur], bytes, hipMemcpyDeviceToDevice, st), kCtx);
   return rc;
 }
