@@ -430,7 +430,8 @@ constexpr int kBinRows = 512;          // blocks that bin the particles, at most
 constexpr int kRowCols = 16;           // bricks per block of scan_rows
 constexpr int kRowSegments = 64;
 constexpr int kMaxBricks = 16384;      // 64 KB of LDS counters
-constexpr int kBrickTarget = 512;      // particles per brick aimed at
+constexpr int kBrickTarget = 512;      // particles per brick of up to 256 cells, at most
+constexpr int kThinTarget = 128;       // of a larger one
 constexpr int kMostGroup = 32;         // records of one block in one brick
 // Particles per cell of the window: denser sets are sorted, since a cell's thread walks
 // its contributions alone (1M particles on 24^3 cells, 72 per cell: 1250 us by bricks,
@@ -767,15 +768,27 @@ SumBricksFn sum_bricks_fn(int cells, int* threads)
                         : sum_bricks<256, 4, 128>;
 }
 
-// Brick shape for np particles on the window: about kBrickTarget particles per
-// brick, within 64 to 1024 cells (fewer on windows of fewer resolved axes) and
-// kMaxBricks bricks.  False where that many bricks do not cover the window.
+// Brick shape for np particles on the window, within 64 to 1024 cells (fewer on windows
+// of fewer resolved axes) and kMaxBricks bricks: up to 256 cells for at most kBrickTarget
+// particles per brick, more for at most kThinTarget.  A cell thread of a larger brick
+// holds 2 or 4 cells whose masks it walks one after the other, which pays only where
+// there is little in them (per call, 256, 512 and 1024 cells: 1M particles on 128^3 212,
+// 217 and 257 us, 100k on 64^3 69, 81 and 108; 500k on 160x160x80 155, 142 and 160, 200k on
+// 128^3 124, 110 and 104).  False where kMaxBricks bricks do not cover the window.
 bool choose_bricks(const CellGrid& g, const Coords& pc, int64_t np, Bricks* b)
 {
   const double window = (double)g.nmax[0] * g.nmax[1] * g.nmax[2];
-  if (np > kMostPerCell * window) return false;
+  // A brick's time goes with the particles per cell, the sort's with the particles: small
+  // dense sets are sorted (per call, bricks and sort: 200k particles on 24^3 366 and 244 us,
+  // 20k on 16^3 203 and 155, 8k on 12^3 175 and 132; 400k on 30^3 317 and 340, 200k 188 and
+  // 226, 500k on 40^3 198 and 413), less soon where an axis has one cell or is not resolved
+  // and a particle reaches fewer cells (60k on 100x60 140 and 190, 150k 278 and 261).
+  double per_cell = np / window;
+  for (int a = 0; a < 3; ++a)
+    if (!pc.c[a] || g.nmax[a] == 1) per_cell *= 0.4;
+  if (np > kMostPerCell * window || per_cell > 2.6 + np / 35000.0) return false;
   int bits = 6;
-  while (bits < 10 && np / window * (double)(2 << bits) <= kBrickTarget) ++bits;
+  while (bits < 10 && np / window * (double)(2 << bits) <= (bits < 8 ? kBrickTarget : kThinTarget)) ++bits;
   for (;; ++bits) {
     int used = 0;
     for (int a = 0; a < 3; ++a) b->sh[a] = 0;
@@ -832,10 +845,12 @@ int scatter_by_bricks(double* dest, const double* src, const CellGrid& g, const 
   *counted = *done = false;
   Bricks b;
   if (np >= (int64_t(1) << 31) || !choose_bricks(g, pc, np, &b)) return NEBO_OK;
-  // at most kBinRows rows, more where the bricks are few (dense sets), so that one
-  // block's records of one brick stay few
+  // a row per 1024 particles, and per 4 particles per brick, so that one block's records
+  // of one brick stay few (5000 particles on 24^3 cells, 54 bricks: rows of 1000 left the
+  // set to the sort, 150 us); at most kBinRows, more where the bricks are few (dense sets)
   const int64_t most_rows = std::max<int64_t>(kBinRows, (int64_t)kBinRows * 4096 / b.total);
-  const int n_rows = (int)std::min<int64_t>(most_rows, (np + 1023) / 1024);
+  const int64_t rows_wanted = std::max((np + 1023) / 1024, np / (4 * (int64_t)b.total));
+  const int n_rows = (int)std::min<int64_t>(most_rows, rows_wanted);
   const int share = (int)((np + n_rows - 1) / n_rows);
   const size_t row_bytes = sizeof(uint32_t) * (size_t)b.total;
   char* work = nullptr;

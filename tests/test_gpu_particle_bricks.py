@@ -127,3 +127,15 @@ def test_gather_of_every_span(axes, edge, spacing):
         want = orc.cell_to_particle(cells, *coords, size, geom, m)
     assert np.array_equal(out.cpu().numpy(), want, equal_nan=True)
     assert skipped.item() > 0
+
+
+@pytest.mark.parametrize("n,npart", [((16, 16, 16), 1000), ((24, 24, 24), 5000), ((32, 32, 32), 20000),
+                                     ((160, 30, 10), 300), ((60, 50, 40), 20000), ((16, 16, 16), 20000),
+                                     ((100, 60, 1), 60000), ((12, 12, 12), 8000)])
+def test_brick_sizes_and_the_line_to_the_sort(n, npart):
+    """Rows of fewer than 1024 particles, bricks of 64 to 1024 cells, and sets on both
+    sides of the line past which they are sorted."""
+    L = nh.Layout.build(n, 1)
+    rng = np.random.default_rng(npart + n[0])
+    box = [(0.0, float(e)) for e in n]
+    scatter(L, *cloud(rng, npart, box, 0.2, 1.5), (1.0, 0.5, 1.0, 0.5, 1.0, 0.5))
