@@ -175,7 +175,8 @@ int nebo_init(int device);
  * reuse (replaces Pool<T>::get/put, spatialops/structured/MemoryPool.cpp:102-186). */
 int nebo_alloc(int device, size_t bytes, void** out);
 int nebo_free(int device, void* ptr);
-/* Release every pooled block of `device` back to the runtime. */
+/* Release every pooled block of `device`, and the scratch blocks kept between calls,
+ * back to the runtime. */
 int nebo_pool_trim(int device);
 /* Bytes currently handed out / high-water mark (MemoryPool.h:49,82-90). */
 int nebo_pool_stats(int device, size_t* in_use, size_t* high_water);
@@ -426,13 +427,16 @@ int nebo_lapl_euler(const nebo_field_t* out, const nebo_field_t* phi,
  *   2. else the tile nebo_stencil_autotune found fastest for a box of the same
  *      dimensions on the same device;
  *   3. else 128 x 8 tiles, variant 7, with the longest z chunk of 512, 256 or
- *      128 planes that gives every CU a workgroup (512^3: 512 planes);
+ *      128 planes that gives every CU a workgroup (512^3: 512 planes), where the
+ *      box is a multiple of the tile in x and y or holds 66 % of the cells that
+ *      whole rounds of one tile per CU could;
  *   4. else 128 x 8 x 64, variant 11 for kernel 0 on boxes whose width is a
- *      multiple of 128 and variant 7 otherwise, when it gives at least half the
- *      device's CUs a workgroup (256^3);
- *   5. else (small boxes) variant 3 with 64 x 2 tiles (one wave, 2 rows per
- *      lane) and the longest z chunk of 16, 8 or 4 planes that gives the device
- *      two workgroups per CU, else 4 planes.
+ *      multiple of 128 and variant 7 otherwise, where the box holds 66 % of those
+ *      cells (256^3);
+ *   5. else variant 3 with one-wave tiles: 64 x 4 (4 rows per lane) and 8 planes on
+ *      boxes that give a CU 24 (kernel 1: 44) workgroups of 64 x 2 and 8 planes;
+ *      below, 64 x 2 and 8 planes down to 16 of them, 16 planes where that gives a
+ *      CU 4 workgroups, 8 planes likewise, else 4.
  * nebo_stencil_set_tile with tx = ty = zchunk = variant = 0 removes the pin.
  * nebo_stencil_get_tile reports the tile last pinned or tuned (the default tile
  * if neither).  The tile changes only the schedule, never the results.  The
@@ -570,11 +574,12 @@ int nebo_diffusion_backward(const nebo_field_t* lam0, double* gk,
  * lane exchange, y neighbours from the lane's rows) with loads 2 planes ahead,
  * 3 the same with loads 1 plane ahead.  By box size: column tiles with loads 1
  * plane ahead and the longest z chunk of 512, 256, 128 or 64 planes that gives
- * every CU a workgroup, else the direct schedule.  zchunk: planes per workgroup, 0 for the schedule's
- * default (16 for the direct one).  The adjoint stage always runs the direct
- * schedule (a zchunk set with schedule 1 applies to it).  Changes only the
- * schedule, never the results.  nebo_transport_schedule reports the schedule
- * and chunk a stage over `field`'s interior would use.  No reference
+ * every CU a workgroup, where the box fills them; one-wave column tiles on boxes
+ * of many such waves (the adjoint stage on mid-size ones too); else the direct
+ * schedule.  zchunk: planes per workgroup, 0 for the schedule's default (16 for
+ * the direct one, fewer on boxes that leave CUs idle).  Both stages follow it.
+ * Changes only the schedule, never the results.  nebo_transport_schedule reports
+ * the schedule and chunk a stage over `field`'s interior would use.  No reference
  * counterpart. */
 int nebo_transport_tune(int32_t schedule, int32_t zchunk);
 int nebo_transport_schedule(const nebo_field_t* field, int32_t* schedule, int32_t* zchunk);
@@ -640,9 +645,11 @@ typedef struct nebo_particle_geom {
  * adds src[p] * (its volume fraction in the cell) to every cell of dest it
  * overlaps.  px / py / pz may be NULL for an axis the particles do not resolve.
  * Every cell receives its contributions in particle order, so the sums are those
- * of the reference's serial loop bit for bit: the contributions, written in the
- * serial loop's order, are stably sorted by cell and summed per cell.  A particle whose box begins a cell or
- * more below the window on some axis contributes nothing (the reference's
+ * of the reference's serial loop bit for bit: the particles are listed per brick
+ * of cells and each cell adds its contributions in their order (sets crowded into
+ * few cells: the contributions are stably sorted by cell).  The call waits on the
+ * stream once, for the number of list entries.  A particle whose box begins a cell
+ * or more below the window on some axis contributes nothing (the reference's
  * unsigned index conversion wraps there); `skipped` (device int, may be NULL)
  * receives how many did.  All particle arrays hold np doubles on dest's GPU. */
 int nebo_particle_to_cell(const nebo_field_t* dest, const double* src, const double* px,
