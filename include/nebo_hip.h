@@ -436,7 +436,9 @@ int nebo_lapl_euler(const nebo_field_t* out, const nebo_field_t* phi,
  *   5. else variant 3 with one-wave tiles: 64 x 4 (4 rows per lane) and 8 planes on
  *      boxes that give a CU 24 (kernel 1: 44) workgroups of 64 x 2 and 8 planes;
  *      below, 64 x 2 and 8 planes down to 16 of them, 16 planes where that gives a
- *      CU 4 workgroups, 8 planes likewise, else 4.
+ *      CU 4 workgroups, 8 planes likewise, else 4.  (nebo_diffusion_step and the
+ *      trajectories, whose launches also write ghost images, take 8 planes for 16
+ *      below 6 workgroups per CU.)
  * nebo_stencil_set_tile with tx = ty = zchunk = variant = 0 removes the pin.
  * nebo_stencil_get_tile reports the tile last pinned or tuned (the default tile
  * if neither).  The tile changes only the schedule, never the results.  The

@@ -896,8 +896,10 @@ double tile_fill(int shape, const nebo_limits_t& lim, int cus)
   return cells / ((double)rounds * cus * sh.tx * tile_geometry(sh).tile_y * sh.zc);
 }
 
-int select_shape(int kernel, int device, const nebo_limits_t& lim)
+// by_rule (if any): whether the size rule chose it, not a pinned or tuned tile.
+int select_shape(int kernel, int device, const nebo_limits_t& lim, bool* by_rule = nullptr)
 {
+  if (by_rule) *by_rule = false;
   const int pinned = g_pinned[kernel].load();
   if (pinned >= 0) return pinned;
   const int n[3] = {lim.hi[0] - lim.lo[0], lim.hi[1] - lim.lo[1], lim.hi[2] - lim.lo[2]};
@@ -907,6 +909,7 @@ int select_shape(int kernel, int device, const nebo_limits_t& lim)
       if (t.kernel == kernel && t.device == device && t.n[0] == n[0] && t.n[1] == n[1] && t.n[2] == n[2])
         return t.shape;
   }
+  if (by_rule) *by_rule = true;
   const int cus = device_cu_count(device);
   const TileShape def = kShapes[kDefaultShape];
   const bool divides = n[0] % def.tx == 0 && n[1] % tile_geometry(def).tile_y == 0;
@@ -1117,8 +1120,15 @@ int launch_diffusion_euler(const nebo_field_t* out, const nebo_field_t* k, const
                            const nebo_axis_coefs_t& c, double dt, void* stream)
 {
   const nebo_limits_t lim = interior_of(out);
-  const int shape = usable_shape(select_shape(0, out->device, lim), out->glob[0], out->glob[0] * out->glob[1],
-                                 lim.hi[0] - lim.lo[0], 0);
+  bool by_rule = false;
+  int pick = select_shape(0, out->device, lim, &by_rule);
+  // walks of 8 planes for 16 on boxes of few waves, where those that write ghost images set
+  // the time (per step of 20, the input's fill included: 128^3, 4 waves of 16 planes per CU,
+  // 17.4 us against 18.7, 112x150x130, 5.3, 19.8 and 21.9; 256x128x100, 7, 23.6 and 23.2,
+  // 180x150x130, 7.9, 24.5 and 24.1)
+  if (by_rule && pick == kSmallColumn[0] && tile_groups(pick, lim) < 6L * device_cu_count(out->device))
+    pick = kSmallColumn[1];
+  const int shape = usable_shape(pick, out->glob[0], out->glob[0] * out->glob[1], lim.hi[0] - lim.lo[0], 0);
   const int rc = launch_divk_shape(shape, 2, out, k, phi, c, dt, lim, stream);
   if (rc) return rc;
   return writes_images(kShapes[shape]) ? fill_thin_ghosts(out, stream) : fill_ghosts_periodic(out, stream);

@@ -94,3 +94,16 @@ def test_ghost_fill_of_uneven_layers(n, ghost):
     nh.fill_ghosts_periodic(f)
     orc.fill_periodic(f)
     assert same(f.gpu, f.host)
+
+
+@pytest.mark.parametrize("n", [(112, 150, 130), (256, 128, 100)])
+def test_diffusion_step_of_8_and_16_planes(n):
+    """Boxes on which the size rule gives 16 planes and the step takes 8, and 16."""
+    L, rng = layout(n), np.random.default_rng(sum(n))
+    c = nh.axis_coefs(nh.build_stencils(7, 11, 13, 1.0, 1.0, 1.0))
+    phi, k, zero = block(n, rng), block(n, rng, 0.5, 2.0), np.zeros(L.npts)
+    want, out = nh.Field(L, host=zero.copy()), dev(zero)
+    orc.diffusion_step(want, nh.Field(L, host=phi), nh.Field(L, host=k), c, 1e-4)
+    adj.diffusion_step(L, out, dev(phi), dev(k), c, 1e-4)
+    assert nh.stencil_select_tile(0, n) == (64, 2, 16, 3)
+    assert same(out, want.host)
