@@ -223,7 +223,9 @@ __device__ __forceinline__ bool particle_range(const CellGrid& g, const bool (&h
     r->lo[a] = (int)(t > 2147483646.0 ? 2147483646.0 : (t > 0.0 ? t : 0.0));
     if (has[a]) {
       double u = divide(r->plo[a] + v.size - g.loface[a], g.h[a], g.rh[a], safe);
-      u = u > 2147483646.0 ? 2147483646.0 : (u < -2.0e9 ? -2.0e9 : u);
+      // an end below the window (a cube of negative size, or NaN) is 0: lo >= 0, so the
+      // range is empty, and hi - lo cannot pass the range of an int
+      u = u > 2147483646.0 ? 2147483646.0 : (u > -1.0 ? u : -1.0);
       r->hi[a] = (int)u + 1;
     } else {
       r->hi[a] = r->lo[a] + 1;
