@@ -266,5 +266,13 @@ int check_hip(int hip_status, const char* ctx);
 // captured, and for blocks larger than the cache may keep).
 int scratch_alloc(void** out, size_t bytes, void* stream, const char* ctx);
 void scratch_free(void* p, void* stream);
+// Gives the idle scratch blocks of a device, and the idle slots below, back.
+void scratch_trim(int device);
+
+// A page-locked slot of kHostSlotBytes bytes that kernels can write results to which
+// the host reads after a synchronisation; one per call in progress.
+constexpr size_t kHostSlotBytes = 64;
+int host_slot_take(void** out, const char* ctx);
+void host_slot_give(void* p);
 
 }  // namespace nebo

@@ -32,7 +32,6 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <mutex>
 #include <unordered_map>
 #include <vector>
 
@@ -425,6 +424,7 @@ struct BrickStats {
   uint32_t most;      // of the fullest brick
   uint32_t group;     // that one block writes into one brick, at most
 };
+static_assert(sizeof(BrickStats) <= kHostSlotBytes, "statistics are written to a slot");
 
 constexpr int kBinThreads = 512;
 constexpr int kBinBatch = 4;          // particles a thread loads at a time
@@ -815,27 +815,6 @@ bool choose_bricks(const CellGrid& g, const Coords& pc, int64_t np, Bricks* b)
   }
 }
 
-// Page-locked slots the statistics are written to, one per call in progress.
-std::mutex g_stats_mu;
-std::vector<BrickStats*> g_stats_free;
-
-int take_stats(BrickStats** s, const char* ctx)
-{
-  std::lock_guard<std::mutex> lk(g_stats_mu);
-  if (!g_stats_free.empty()) {
-    *s = g_stats_free.back();
-    g_stats_free.pop_back();
-    return NEBO_OK;
-  }
-  return check_hip(hipHostMalloc((void**)s, sizeof(BrickStats), hipHostMallocPortable | hipHostMallocMapped), ctx);
-}
-
-void give_stats(BrickStats* s)
-{
-  std::lock_guard<std::mutex> lk(g_stats_mu);
-  g_stats_free.push_back(s);
-}
-
 // The scatter by bricks.  *counted: the particles were counted (and the skipped ones
 // reported); *done: dest holds the sums.  Left to the sort when *done stays false:
 // windows of too many bricks, and sets crowded into few bricks (more than
@@ -857,12 +836,12 @@ int scatter_by_bricks(double* dest, const double* src, const CellGrid& g, const 
   const size_t row_bytes = sizeof(uint32_t) * (size_t)b.total;
   char* work = nullptr;
   BrickStats* stats = nullptr;
-  int rc = take_stats(&stats, ctx);
+  int rc = host_slot_take((void**)&stats, ctx);
   if (rc) return rc;
   // rows, totals, base (+1), group (one per block of scan_rows)
   const int n_group = (b.total + kRowCols - 1) / kRowCols;
   if ((rc = scratch_alloc((void**)&work, row_bytes * (n_rows + 2) + sizeof(uint32_t) * (1 + n_group), s, ctx))) {
-    give_stats(stats);
+    host_slot_give(stats);
     return rc;
   }
   uint32_t* rows = reinterpret_cast<uint32_t*>(work);
@@ -879,7 +858,7 @@ int scatter_by_bricks(double* dest, const double* src, const CellGrid& g, const 
   rc = check_hip(hipGetLastError(), ctx);
   if (!rc) rc = check_hip(hipStreamSynchronize(s), ctx);
   const BrickStats st = *stats;
-  give_stats(stats);
+  host_slot_give(stats);
   if (rc) {
     scratch_free(work, s);
     return rc;
