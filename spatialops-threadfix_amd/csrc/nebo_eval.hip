@@ -893,8 +893,7 @@ extern "C" int nebo_masked_assign(const nebo_field_t* lhs, const int32_t* points
   hipStream_t s = (hipStream_t)stream;
   int32_t* pts = nullptr;
   const size_t bytes = sizeof(int32_t) * 3 * (size_t)n_points;
-  if ((rc = scratch_alloc((void**)&pts, bytes, s, ctx))) return rc;
-  if ((rc = check_hip(hipMemcpyAsync(pts, points, bytes, hipMemcpyHostToDevice, s), ctx))) return rc;
+  if ((rc = scratch_upload((void**)&pts, points, bytes, s, ctx))) return rc;
   dim3 grid((n_points + kBlock - 1) / kBlock);
   const bool one = prog.n_classes == 1, math = uses_math(prog);
   BackendScope bs("masked assignment (" + std::to_string(n_points) + " points)");

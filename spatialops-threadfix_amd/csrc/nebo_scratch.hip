@@ -162,6 +162,18 @@ void scratch_free(void* p, void* stream)
   scratch_evict(c, c.limit);   // blocks lent together may have passed the limit
 }
 
+int scratch_upload(void** out, const void* host, size_t bytes, void* stream, const char* ctx)
+{
+  int rc = scratch_alloc(out, bytes, stream, ctx);
+  if (rc) return rc;
+  rc = check_hip(hipMemcpyAsync(*out, host, bytes, hipMemcpyHostToDevice, (hipStream_t)stream), ctx);
+  if (rc) {
+    scratch_free(*out, stream);
+    *out = nullptr;
+  }
+  return rc;
+}
+
 void scratch_trim(int device)
 {
   const RelaxedCapture relaxed;

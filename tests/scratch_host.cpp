@@ -105,6 +105,12 @@ hipError_t hipEventQuery(hipEvent_t e)
 }
 hipError_t hipEventSynchronize(hipEvent_t e) { finish(((Event*)e)->stream); return hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t, unsigned) { ++streams[s].queued; return hipSuccess; }
+hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t s)
+{
+  if (fail_copy) return hipErrorInvalidValue;
+  ++streams[s].queued;
+  return hipSuccess;
+}
 hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t* p, int) { *p = nullptr; return hipSuccess; }
 hipError_t hipMemPoolTrimTo(hipMemPool_t, size_t) { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "error"; }
@@ -146,10 +152,24 @@ static void slots_are_reused()
   CHECK(host_bytes == 0);
 }
 
+// A copy that fails holds no block: a trim leaves nothing allocated.
+static void failed_upload()
+{
+  const int host[4] = {1, 2, 3, 4};
+  void* p = nullptr;
+  CHECK(scratch_upload(&p, host, sizeof host, A, "t") == NEBO_OK && p);
+  scratch_free(p, A);
+  fail_copy = true;
+  CHECK(scratch_upload(&p, host, sizeof host, A, "t") == NEBO_ERR_HIP && !p);
+  scratch_trim(0);
+  CHECK(used == 0);
+}
+
 int main(int argc, char** argv)
 {
   const struct { const char* name; void (*fn)(); } checks[] = {
-      {"other_threads_capture", other_threads_capture}, {"slots_are_reused", slots_are_reused}};
+      {"other_threads_capture", other_threads_capture}, {"slots_are_reused", slots_are_reused},
+      {"failed_upload", failed_upload}};
   for (const auto& c : checks)
     if (argc == 2 && !std::strcmp(argv[1], c.name)) {
       c.fn();
