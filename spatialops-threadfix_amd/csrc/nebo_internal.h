@@ -263,7 +263,8 @@ int check_hip(int hip_status, const char* ctx);
 // Scratch memory of one call on the current device, usable by work queued on
 // `stream` until scratch_free gives it back in that stream's order: from a bounded
 // cache of blocks (from the runtime's stream-ordered pool while the stream is
-// captured, and for blocks larger than the cache may keep).
+// captured, and where the block would pass what the cache may keep).  Neither waits on
+// the host for other work, unless memory runs out.
 int scratch_alloc(void** out, size_t bytes, void* stream, const char* ctx);
 void scratch_free(void* p, void* stream);
 // scratch_alloc of a copy of `bytes` bytes of host memory; nothing is held on failure.

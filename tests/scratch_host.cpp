@@ -111,7 +111,7 @@ hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t
   ++streams[s].queued;
   return hipSuccess;
 }
-hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t* p, int) { *p = nullptr; return hipSuccess; }
+hipError_t hipDeviceGetMemPool(hipMemPool_t* p, int) { *p = nullptr; return hipSuccess; }
 hipError_t hipMemPoolTrimTo(hipMemPool_t, size_t) { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "error"; }
 }
@@ -165,11 +165,108 @@ static void failed_upload()
   CHECK(used == 0);
 }
 
+static constexpr size_t MB = size_t(1) << 20;
+
+static void* get(size_t bytes, void* stream)
+{
+  void* p = nullptr;
+  CHECK(scratch_alloc(&p, bytes, stream, "t") == NEBO_OK && p);
+  return p;
+}
+
+// Blocks given back, of whatever sizes and streams, never pass 1/32 of the memory, and
+// neither taking nor giving waits on the host, with all of the streams' work undone.
+static void kept_within_the_limit()
+{
+  for (int i = 0; i < 40; ++i) {
+    void* s = i % 2 ? A : B;
+    void* p = get((100 + 90 * i) * MB, s);   // the largest pass the limit of 2048 MB
+    scratch_free(p, s);
+    CHECK(used <= total / 32);
+  }
+  CHECK(waits == 0);
+}
+
+// Blocks lent at one time may pass the limit; those past it are not kept.
+static void lent_together()
+{
+  std::vector<void*> p;
+  for (int i = 0; i < 8; ++i) p.push_back(get(500 * MB, A));
+  CHECK(used >= 4000 * MB);
+  for (void* q : p) scratch_free(q, A);
+  CHECK(used <= total / 32 && used >= 1500 * MB);
+  CHECK(waits == 0);
+}
+
+// The limit follows what others leave free.
+static void little_memory_left()
+{
+  used = total - 4096 * MB;      // another program's
+  const size_t others = used;
+  void* p = get(400 * MB, A);
+  scratch_free(p, A);
+  CHECK(used - others == 416 * MB && get(400 * MB, A) == p);   // in steps of 32 MB
+  scratch_free(p, A);
+  p = get(600 * MB, A);          // more than an eighth of 4096 MB
+  scratch_free(p, A);
+  CHECK(used - others <= 512 * MB);
+  CHECK(waits == 0);
+}
+
+// Another stream's block whose work is not over is taken only where a new one would pass
+// the limit, and then after a wait queued on the taking stream.
+static void blocks_between_streams()
+{
+  void* p = get(1500 * MB, A);
+  scratch_free(p, A);
+  CHECK(get(1500 * MB, A) == p);           // its own stream: at once
+  scratch_free(p, A);
+  void* small = get(400 * MB, B);
+  CHECK(small != p);                        // fits the block, but a new one fits the limit
+  scratch_free(small, B);
+  const long before = streams[B].queued;
+  CHECK(get(1400 * MB, B) == p && streams[B].queued > before);
+  scratch_free(p, B);
+  CHECK(waits == 0);
+  streams[B].done = streams[B].queued;
+  CHECK(get(1500 * MB, A) == p);           // its last use is over
+}
+
+// When memory runs out, what is kept idle goes, and the call succeeds.
+static void memory_runs_out()
+{
+  void* p = get(1024 * MB, A);
+  scratch_free(p, A);
+  used = total - 300 * MB;                  // others took the rest
+  void* q = get(1200 * MB, B);
+  CHECK(live.count(p) == 0 && used == total - 300 * MB - 1024 * MB + 1200 * MB);
+  scratch_free(q, B);
+  CHECK(used == total - 300 * MB - 1024 * MB);
+  void* r = nullptr;
+  used = total;
+  CHECK(scratch_alloc(&r, 600 * MB, A, "t") == NEBO_ERR_HIP && !r);
+}
+
+// A captured stream takes the graph's own allocation nodes.
+static void captured_stream()
+{
+  void* p = get(10 * MB, A);
+  scratch_free(p, A);
+  captured = B;
+  void* q = get(10 * MB, B);
+  CHECK(q != p);
+  scratch_free(q, B);
+  CHECK(live.count(q) == 0 && live.count(p) == 1);
+}
+
 int main(int argc, char** argv)
 {
   const struct { const char* name; void (*fn)(); } checks[] = {
       {"other_threads_capture", other_threads_capture}, {"slots_are_reused", slots_are_reused},
-      {"failed_upload", failed_upload}};
+      {"failed_upload", failed_upload}, {"kept_within_the_limit", kept_within_the_limit},
+      {"lent_together", lent_together}, {"little_memory_left", little_memory_left},
+      {"blocks_between_streams", blocks_between_streams}, {"memory_runs_out", memory_runs_out},
+      {"captured_stream", captured_stream}};
   for (const auto& c : checks)
     if (argc == 2 && !std::strcmp(argv[1], c.name)) {
       c.fn();
