@@ -319,7 +319,7 @@ int build_items(nebo_batch* b)
   }
   b->d_items = nullptr;
   b->n_items = (int)items.size();
-  int rc = check_hip(hipMalloc((void**)&b->d_items, sizeof(int4) * std::max<size_t>(1, items.size())), ctx);
+  int rc = device_alloc((void**)&b->d_items, sizeof(int4) * std::max<size_t>(1, items.size()), ctx);
   if (rc) return rc;
   rc = check_hip(hipMemcpy(b->d_items, items.data(), sizeof(int4) * items.size(), hipMemcpyHostToDevice), ctx);
   if (rc) return rc;
@@ -463,7 +463,7 @@ extern "C" int nebo_batch_create(const nebo_patch_t* patches, int32_t n, const n
     d.XY = d.X * (p.n[1] + 2);
     d.origin = 1 + d.X + d.XY;
   }
-  if (!rc) rc = check_hip(hipMalloc((void**)&b->d_patches, sizeof(DevPatch) * n), ctx);
+  if (!rc) rc = device_alloc((void**)&b->d_patches, sizeof(DevPatch) * n, ctx);
   if (!rc) rc = check_hip(hipMemcpy(b->d_patches, dp.data(), sizeof(DevPatch) * n, hipMemcpyHostToDevice), ctx);
   if (!rc) rc = build_items(b);
   if (rc) {

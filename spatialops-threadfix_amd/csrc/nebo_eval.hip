@@ -765,7 +765,7 @@ int stream_reduce_buffer(void* stream, StreamRedBuf* out)
     return NEBO_OK;
   }
   char* p = nullptr;
-  if ((rc = check_hip(hipMalloc((void**)&p, kRedBufBytes), ctx))) return rc;
+  if ((rc = device_alloc((void**)&p, kRedBufBytes, ctx))) return rc;
   StreamRedBuf b{red_buf_at(p), new std::mutex};
   g_redbuf[key] = b;
   *out = b;

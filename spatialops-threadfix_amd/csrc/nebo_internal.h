@@ -269,6 +269,8 @@ int scratch_alloc(void** out, size_t bytes, void* stream, const char* ctx);
 void scratch_free(void* p, void* stream);
 // scratch_alloc of a copy of `bytes` bytes of host memory; nothing is held on failure.
 int scratch_upload(void** out, const void* host, size_t bytes, void* stream, const char* ctx);
+// hipMalloc on the current device; its idle scratch blocks go when there is no memory.
+int device_alloc(void** out, size_t bytes, const char* ctx);
 // Gives the idle scratch blocks of a device, and the idle slots below, back.
 void scratch_trim(int device);
 

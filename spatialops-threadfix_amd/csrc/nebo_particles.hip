@@ -1093,7 +1093,7 @@ extern "C" int nebo_point_map_create(const int64_t* indices, int64_t n, int devi
   m->gather = m->scatter_src = m->scatter_dst = nullptr;
   const size_t b1 = sizeof(int64_t) * (size_t)n, b2 = sizeof(int64_t) * from.size();
   if (n > 0) {
-    rc = check_hip(hipMalloc((void**)&m->gather, b1 + 2 * b2), ctx);
+    rc = device_alloc((void**)&m->gather, b1 + 2 * b2, ctx);
     if (!rc) {
       m->scatter_src = m->gather + n;
       m->scatter_dst = m->scatter_src + m->m;

@@ -302,7 +302,7 @@ extern "C" int nebo_alloc(int device, size_t bytes, void** out)
     it->second.pop_back();
   } else {
     int rc = with_device(device, "Nebo Memory", [&] {
-      return check_hip(hipMalloc(&p, bytes), "Nebo Memory");
+      return device_alloc(&p, bytes, "Nebo Memory");
     });
     if (rc) return rc;
   }

@@ -226,6 +226,19 @@ int scratch_upload(void** out, const void* host, size_t bytes, void* stream, con
   return rc;
 }
 
+int device_alloc(void** out, size_t bytes, const char* ctx)
+{
+  int device = 0;
+  int rc = check_hip(hipGetDevice(&device), ctx);
+  if (rc) return rc;
+  hipError_t st = hipMalloc(out, bytes);
+  if (st == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    if (scratch_drop(device)) st = hipMalloc(out, bytes);
+  }
+  return check_hip(st, ctx);
+}
+
 void scratch_trim(int device)
 {
   (void)scratch_drop(device);

@@ -247,6 +247,17 @@ static void memory_runs_out()
   CHECK(scratch_alloc(&r, 600 * MB, A, "t") == NEBO_ERR_HIP && !r);
 }
 
+// The same for memory a program allocates to keep.
+static void program_memory_runs_out()
+{
+  void* p = get(1024 * MB, A);
+  scratch_free(p, A);
+  used = total - 300 * MB;
+  void* q = nullptr;
+  CHECK(device_alloc(&q, 1200 * MB, "t") == NEBO_OK && q && live.count(p) == 0);
+  CHECK(device_alloc(&q, 1200 * MB, "t") == NEBO_ERR_HIP);
+}
+
 // A captured stream takes the graph's own allocation nodes.
 static void captured_stream()
 {
@@ -266,7 +277,7 @@ int main(int argc, char** argv)
       {"failed_upload", failed_upload}, {"kept_within_the_limit", kept_within_the_limit},
       {"lent_together", lent_together}, {"little_memory_left", little_memory_left},
       {"blocks_between_streams", blocks_between_streams}, {"memory_runs_out", memory_runs_out},
-      {"captured_stream", captured_stream}};
+      {"program_memory_runs_out", program_memory_runs_out}, {"captured_stream", captured_stream}};
   for (const auto& c : checks)
     if (argc == 2 && !std::strcmp(argv[1], c.name)) {
       c.fn();

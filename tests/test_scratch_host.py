@@ -10,7 +10,8 @@ import pytest
 HERE = os.path.dirname(os.path.abspath(__file__))
 SOURCE = os.path.join(HERE, "..", "spatialops-threadfix_amd", "csrc", "nebo_scratch.hip")
 CHECKS = ["other_threads_capture", "slots_are_reused", "failed_upload", "kept_within_the_limit", "lent_together",
-          "little_memory_left", "blocks_between_streams", "memory_runs_out", "captured_stream"]
+          "little_memory_left", "blocks_between_streams", "memory_runs_out", "program_memory_runs_out",
+          "captured_stream"]
 
 pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not installed")
 
