@@ -648,9 +648,10 @@ typedef struct nebo_particle_geom {
  * overlaps.  px / py / pz may be NULL for an axis the particles do not resolve.
  * Every cell receives its contributions in particle order, so the sums are those
  * of the reference's serial loop bit for bit: the particles are listed per brick
- * of cells and each cell adds its contributions in their order (sets crowded into
- * few cells: the contributions are stably sorted by cell).  The call waits on the
- * stream once, for the number of list entries.  A particle whose box begins a cell
+ * of cells and each cell adds its contributions in their order (sets dense in or
+ * crowded into few cells: the contributions are stably sorted by cell).  The call
+ * waits on the stream for the number of list entries, of sorted contributions
+ * likewise, and of both where the list shows that a set is crowded.  A particle whose box begins a cell
  * or more below the window on some axis contributes nothing (the reference's
  * unsigned index conversion wraps there); `skipped` (device int, may be NULL)
  * receives how many did.  All particle arrays hold np doubles on dest's GPU. */

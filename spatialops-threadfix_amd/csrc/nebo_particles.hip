@@ -7,8 +7,8 @@
 // loop bit for bit (ParticleOperators.h:184-270), so atomics on the cells are out.
 // The scatter by bricks (below, "ParticleToCell by bricks") gathers the particles of
 // one brick of cells in LDS and puts each cell's contributions in particle order
-// there.  Particle sets it does not suit (very many particles in one brick) are
-// sorted in device memory:
+// there.  Particle sets it does not suit (dense in the window, or crowded into a few
+// bricks of it) are sorted in device memory:
 //   1. count the cells each particle overlaps, exclusive scan -> entry offsets;
 //   2. each particle writes its entries in its own loop order: value
 //      src[p] * fraction and key cell at entry e, so entries stand in the serial
@@ -392,7 +392,9 @@ __global__ void run_sum_kernel(double* __restrict__ dest, const uint32_t* __rest
 //      many of them reach into each brick (one row of counts per block);
 //   2. scan_rows, scan_bricks: places of every block's records of every brick, by
 //      prefix sums over the rows of a brick and over the bricks;
-//   3. fill_bricks: the same blocks write a 48-byte record per particle and brick;
+//   3. fill_bricks: the same blocks write a 48-byte record per particle and brick, or
+//      one wave for each block, where a block has many in one brick (particles in an
+//      order of space);
 //   4. sum_bricks: one workgroup per brick, a thread per cell: the records set their
 //      bits in the masks of the cells they reach, and each cell adds its contributions
 //      in the order of the bits (the serial loop's order).
@@ -400,9 +402,10 @@ __global__ void run_sum_kernel(double* __restrict__ dest, const uint32_t* __rest
 // cells) and by the arithmetic per contribution (75 % of sum_bricks' time issues
 // vector instructions), where a sort of the contributions moves 12 bytes of each (6.3
 // per particle) through memory 7 times.  2M particles of 0.2-1.5 cells on 112x96x104
-// cells: 342 us per call (sum_bricks 140, fill_bricks 118, count_bricks 25, the scans
-// 29) against 870 us sorted; 4M on 128^3: 575 against 1627; 1M on 40^3: 340 against
-// 711.
+// cells: 336 us per call (sum_bricks 131, fill_bricks 128, count_bricks 25, the scans
+// 30) against 870 us sorted; 4M on 128^3: 564 against 1622; 1M on 40^3: 302 against
+// 713.  In cell order 395 against 870 (sum_bricks 188: successive records wait for the
+// same threads; fill_bricks, one wave per block, 132), 4M on 128^3 702 and 1617.
 
 struct Bricks {
   int sh[3];     // log2 of a brick's cells per axis (at most 5)
@@ -434,12 +437,12 @@ constexpr int kRowSegments = 64;
 constexpr int kMaxBricks = 16384;      // 64 KB of LDS counters
 constexpr int kBrickTarget = 512;      // particles per brick of up to 256 cells, at most
 constexpr int kThinTarget = 128;       // of a larger one
-constexpr int kMostGroup = 32;         // records of one block in one brick
+constexpr int kMostGroup = 32;         // records of one block in one brick, in any order
+constexpr int kGranule = 64;           // particles whose records one wave writes at a time
 // Particles per cell of the window: denser sets are sorted, since a cell's thread walks
 // its contributions alone (1M particles on 24^3 cells, 72 per cell: 1250 us by bricks,
 // 700 sorted; on 40^3, 16 per cell: 340 and 711).
 constexpr double kMostPerCell = 32;
-constexpr uint32_t kMostRecords = 1u << 17;   // records of one brick
 
 // f(brick, bx, by, bz) for every brick the range reaches into.
 template <typename F>
@@ -593,48 +596,57 @@ __global__ __launch_bounds__(1024) void scan_bricks(uint32_t* __restrict__ base,
   }
 }
 
-__global__ __launch_bounds__(kBinThreads) void fill_bricks(BrickRec* __restrict__ recs,
-                                                           const uint32_t* __restrict__ rows,
-                                                           const uint32_t* __restrict__ base, CellGrid g, Bricks b,
-                                                           Coords pc, const double* __restrict__ psize,
-                                                           const double* __restrict__ src, long np, int share)
+// NT threads per block.  With kBinThreads a block's records of one brick come out in any
+// order, which sum_bricks puts right where they are few.  With one wave (NT 64) they
+// come out in order up to those of kGranule consecutive particles: a wave's LDS
+// operations are executed one after the other.
+template <int NT>
+__global__ __launch_bounds__(NT) void fill_bricks(BrickRec* __restrict__ recs, const uint32_t* __restrict__ rows,
+                                                  const uint32_t* __restrict__ base, CellGrid g, Bricks b, Coords pc,
+                                                  const double* __restrict__ psize, const double* __restrict__ src,
+                                                  long np, int share)
 {
   extern __shared__ uint32_t bins[];
   const uint32_t* row = rows + (size_t)blockIdx.x * b.total;
-  for (int i = threadIdx.x; i < b.total; i += kBinThreads) bins[i] = base[i] + row[i];
+  for (int i = threadIdx.x; i < b.total; i += NT) bins[i] = base[i] + row[i];
   __syncthreads();
   const long first = (long)blockIdx.x * share, last = min(first + share, np);
-  for (long p0 = first + threadIdx.x; p0 < last; p0 += kBinBatch * kBinThreads) {
+  for (long p0 = first + threadIdx.x; p0 - threadIdx.x < last; p0 += kBinBatch * NT) {
     PIn in[kBinBatch];
     double val[kBinBatch];
 #pragma unroll
     for (int u = 0; u < kBinBatch; ++u) {
-      const long p = min(p0 + u * kBinThreads, last - 1);
+      const long p = min(p0 + u * NT, last - 1);
       in[u] = load_particle(pc, psize, p);
       val[u] = src[p];
     }
 #pragma unroll
     for (int u = 0; u < kBinBatch; ++u) {
-      const long p = p0 + u * kBinThreads;
+      const long p = p0 + u * NT;
       PRange r;
-      if (p >= last || !particle_range(g, b.has, in[u], &r)) continue;
-      BrickRec rec;
+      if (p < last && particle_range(g, b.has, in[u], &r)) {
+        BrickRec rec;
 #pragma unroll
-      for (int a = 0; a < 3; ++a) rec.plo[a] = r.plo[a];
-      rec.size = r.size;
-      rec.src = val[u];
-      rec.idx = (uint32_t)p;
-      for_bricks(b, r, [&](int brick, int x, int y, int z) {
-        const int at[3] = {x, y, z};
-        rec.range = 0;
+        for (int a = 0; a < 3; ++a) rec.plo[a] = r.plo[a];
+        rec.size = r.size;
+        rec.src = val[u];
+        rec.idx = (uint32_t)p;
+        for_bricks(b, r, [&](int brick, int x, int y, int z) {
+          const int at[3] = {x, y, z};
+          rec.range = 0;
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          const int o = at[a] << b.sh[a], m = (1 << b.sh[a]) - 1;
-          const int lo = max(r.lo[a] - o, 0), hi = min(r.hi[a] - 1 - o, m);
-          rec.range |= (uint32_t)(lo | hi << 5) << (10 * a);
-        }
-        recs[atomicAdd(&bins[brick], 1u)] = rec;
-      });
+          for (int a = 0; a < 3; ++a) {
+            const int o = at[a] << b.sh[a], m = (1 << b.sh[a]) - 1;
+            const int lo = max(r.lo[a] - o, 0), hi = min(r.hi[a] - 1 - o, m);
+            rec.range |= (uint32_t)(lo | hi << 5) << (10 * a);
+          }
+          recs[atomicAdd(&bins[brick], 1u)] = rec;
+        });
+      }
+      if constexpr (NT == kGranule) {   // one granule's places before the next one's
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
     }
   }
 }
@@ -656,20 +668,21 @@ __device__ __forceinline__ void for_range(const Bricks& b, uint32_t range, F&& f
 // walks its mask's bits upwards, which is particle order, and adds the contributions
 // it forms from the records.
 //
-// The blocks that wrote the records hold consecutive particles, so a brick's list is
-// in order up to the records one block wrote (at most `group` of them, 1.4 on average
-// in the case above): a record's place follows from its neighbours.  `share` is the
-// particles per block.
+// A brick's list is in order up to the records of one granule, which are at most `group`:
+// a record's place follows from its neighbours.  A granule is what one block of
+// fill_bricks wrote (`share` consecutive particles, 1.4 records on average in the case
+// above), or, where that is much, a part of 2^part of them.
 template <int NT, int Q, int R>
 __global__ __launch_bounds__(NT) void sum_bricks(double* __restrict__ dest, CellGrid g, Bricks b,
                                                  const uint32_t* __restrict__ base,
-                                                 const BrickRec* __restrict__ recs, uint32_t share, int group)
+                                                 const BrickRec* __restrict__ recs, uint32_t share, int part,
+                                                 int group)
 {
   constexpr int C = NT * Q;      // cells, at most
   constexpr int W = R / 64;      // mask words per cell
   __shared__ double plo[3][R], size[R], val[R];
   __shared__ unsigned long long mask[W][C];
-  __shared__ uint32_t idx[R + 4 * (kMostGroup - 1)];
+  __shared__ uint32_t idx[R + 4 * (kGranule - 1)];
 
   const int brick = xcd_tile(blockIdx.x, gridDim.x);
   const uint32_t first = base[brick];
@@ -717,10 +730,12 @@ __global__ __launch_bounds__(NT) void sum_bricks(double* __restrict__ dest, Cell
     for (int i = M + t; i < R + 3 * M; i += NT) {
       const int j = r0 - 2 * M + i;
       if (j < 0 || j >= n) continue;
-      const uint32_t p = idx[i], blk = p / share;
+      // the particles [g0, g0 + gn) are p's granule; "no particle" is in none (p < 2^31)
+      const uint32_t p = idx[i], in = p % share, g0 = p - (in & ((1u << part) - 1));
+      const uint32_t gn = min(1u << part, p - in + share - g0);
       int place = j - r0;
-      for (int k = i - 1; k >= i - M && idx[k] / share == blk; --k) place -= idx[k] > p;
-      for (int k = i + 1; k <= i + M && idx[k] / share == blk; ++k) place += idx[k] < p;
+      for (int k = i - 1; k >= i - M && idx[k] - g0 < gn; --k) place -= idx[k] > p;
+      for (int k = i + 1; k <= i + M && idx[k] - g0 < gn; ++k) place += idx[k] < p;
       if (place < 0 || place >= R) continue;
       const BrickRec r = mine[j];
 #pragma unroll
@@ -759,7 +774,7 @@ __global__ __launch_bounds__(NT) void sum_bricks(double* __restrict__ dest, Cell
     if (at[q] >= 0) dest[at[q]] = acc[q];
 }
 
-using SumBricksFn = void (*)(double*, CellGrid, Bricks, const uint32_t*, const BrickRec*, uint32_t, int);
+using SumBricksFn = void (*)(double*, CellGrid, Bricks, const uint32_t*, const BrickRec*, uint32_t, int, int);
 SumBricksFn sum_bricks_fn(int cells, int* threads)
 {
   *threads = cells <= 64 ? 64 : cells <= 128 ? 128 : 256;
@@ -815,11 +830,31 @@ bool choose_bricks(const CellGrid& g, const Coords& pc, int64_t np, Bricks* b)
   }
 }
 
+// Whether a counted set goes on by bricks, from times in us on MI355X.  The fullest brick's
+// workgroup walks its records alone, the longer for each the fewer waves share them,
+// and much longer where the list is in an order of space, whose successive records belong
+// to the same few cells: per record 0.06 us in bricks of 256 cells in random order, 0.18
+// in cell order, 0.11 and 0.48 in bricks of 64.  A set in random order that is sorted
+// all the same has a clear gain by it (1.25), one in order no loss.  Sets of 5k to 4M
+// particles, some of them crowded into a part of the window, estimated, measured and
+// sorted after the count: 2M in cell order 438, 396 and 917 us, with a fifth of them in
+// 30^3 cells 1440, 1405 and 980; the same at random 714, 698 and 980; 1M on 64^3 in cell
+// order 379, 324 and 605; 1M on 40^3 841, 904 and 737; 30% of 1M random in 20^3 cells 977,
+// 979 and 635.
+bool bricks_pay(const Bricks& b, const BrickStats& st, int64_t np)
+{
+  constexpr double any[] = {0.11, 0.09, 0.06, 0.08, 0.10}, ordered[] = {0.48, 0.28, 0.18, 0.30, 0.30};
+  const int bits = std::max(b.sh[0] + b.sh[1] + b.sh[2], 6) - 6;
+  const bool few = st.group <= kMostGroup;
+  const double rest = st.most - 0.5 * (double)st.records / b.total;
+  const double bricks = 50 + 1e-4 * (double)st.records + (few ? any : ordered)[bits] * rest;
+  return bricks <= (few ? 1.25 : 1.0) * (150 + 4.2e-4 * (double)np);
+}
+
 // The scatter by bricks.  *counted: the particles were counted (and the skipped ones
 // reported); *done: dest holds the sums.  Left to the sort when *done stays false:
-// windows of too many bricks, and sets crowded into few bricks (more than
-// kMostRecords records in one, whose workgroup would walk them alone, or more than
-// kMostGroup of one block in one, which are ordered by comparing neighbours).
+// windows of too many bricks, dense sets, and, after the count (17 us for 5k particles, 40
+// for 2M, 75 for 4M), sets crowded into few bricks.
 int scatter_by_bricks(double* dest, const double* src, const CellGrid& g, const Coords& pc, const double* psize,
                       int64_t np, int32_t* skipped, hipStream_t s, const char* ctx, bool* counted, bool* done)
 {
@@ -864,15 +899,17 @@ int scatter_by_bricks(double* dest, const double* src, const CellGrid& g, const 
     return rc;
   }
   *counted = true;
-  if (st.records > 0 && st.most <= kMostRecords && st.group <= kMostGroup && st.records < (uint64_t(1) << 31)) {
+  if (st.records > 0 && st.records < (uint64_t(1) << 31) && bricks_pay(b, st, np)) {
     BrickRec* recs = nullptr;
     if (!(rc = scratch_alloc((void**)&recs, sizeof(BrickRec) * st.records, s, ctx))) {
-      hipLaunchKernelGGL(fill_bricks, dim3(n_rows), dim3(kBinThreads), row_bytes, s, recs, rows, base, g, b, pc,
-                         psize, src, (long)np, share);
+      const bool few = st.group <= kMostGroup;
+      const auto fill = few ? fill_bricks<kBinThreads> : fill_bricks<kGranule>;
+      hipLaunchKernelGGL(fill, dim3(n_rows), dim3(few ? kBinThreads : kGranule), row_bytes, s, recs, rows, base, g, b,
+                         pc, psize, src, (long)np, share);
       int threads = 0;
       const SumBricksFn fn = sum_bricks_fn(1 << (b.sh[0] + b.sh[1] + b.sh[2]), &threads);
       hipLaunchKernelGGL(fn, dim3(b.total), dim3(threads), 0, s, dest, g, b, base, recs, (uint32_t)share,
-                         (int)st.group);
+                         few ? 31 : 6, few ? (int)st.group : std::min<int>(st.group, kGranule));
       rc = check_hip(hipGetLastError(), ctx);
       scratch_free(recs, s);
     }
