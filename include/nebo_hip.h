@@ -428,11 +428,11 @@ int nebo_lapl_euler(const nebo_field_t* out, const nebo_field_t* phi,
  *      dimensions on the same device;
  *   3. else 128 x 8 tiles, variant 7, with the longest z chunk of 512, 256 or
  *      128 planes that gives every CU a workgroup (512^3: 512 planes), where the
- *      box is a multiple of the tile in x and y or holds 66 % of the cells that
- *      whole rounds of one tile per CU could;
+ *      box holds 77 % of the cells that whole rounds of one tile per CU walk (and
+ *      has 64 planes or is a multiple of the tile in x and y);
  *   4. else 128 x 8 x 64, variant 11 for kernel 0 on boxes whose width is a
- *      multiple of 128 and variant 7 otherwise, where the box holds 66 % of those
- *      cells (256^3);
+ *      multiple of 128 and variant 7 otherwise, where the box holds 66 % of the
+ *      cells that whole rounds of one tile per CU could (256^3);
  *   5. else variant 3 with one-wave tiles: 64 x 4 (4 rows per lane) and 8 planes on
  *      boxes that give a CU 24 (kernel 1: 44) workgroups of 64 x 2 and 8 planes;
  *      below, 64 x 2 and 8 planes down to 16 of them, 16 planes where that gives a

@@ -839,10 +839,8 @@ LaplFn lapl_table(int s) { return lapl_pick(s, std::make_index_sequence<kNumShap
 //     planes ahead) with the longest z chunk (512, 256 or 128 planes) that still
 //     gives every CU a workgroup: one workgroup per CU, all walking the same
 //     planes (512^3 on MI355X: 658 us against 775 us with 64-plane chunks, whose
-//     eight concurrent z slabs lie 135 MB apart), where the tiles fill the CUs (see
-//     kFill) or divide the box in x and y.  (Of the boxes they divide, 384^3 fills
-//     two thirds of the CUs once and leaves the rest idle: 514 us against 320 for
-//     the tile of rule 5; the selection there is one programs rely on.);
+//     eight concurrent z slabs lie 135 MB apart), where the box holds kLongFill of
+//     the cells its rounds of workgroups walk;
 //  4. else the default tile where it fills the CUs (256^3: 64-plane chunks, one
 //     workgroup per CU), for div(k grad phi) on boxes whose width is a multiple of
 //     128 as pair columns;
@@ -887,13 +885,36 @@ long tile_groups(int shape, const nebo_limits_t& lim)
 // against 67.7), 320x256x128 0.63 (72.3 against 61.6).
 constexpr double kFill = 0.66;
 
-double tile_fill(int shape, const nebo_limits_t& lim, int cus)
+double tile_fill(int shape, const nebo_limits_t& lim, int cus, int planes)
 {
   const TileShape sh = kShapes[shape];
   const long groups = tile_groups(shape, lim), rounds = (groups + cus - 1) / cus;
   double cells = 1;
   for (int d = 0; d < 3; ++d) cells *= lim.hi[d] - lim.lo[d];
-  return cells / ((double)rounds * cus * sh.tx * tile_geometry(sh).tile_y * sh.zc);
+  return cells / ((double)rounds * cus * sh.tx * tile_geometry(sh).tile_y * planes);
+}
+
+// The same for the long-chunk tile, by the planes its workgroups walk: a chunk longer
+// than the box costs nothing, a last round of few workgroups costs a whole walk.  In one
+// round, or in filled ones, the long tile is the faster one (div(k grad phi), long chunk
+// and what follows: 512x512x300 385 and 412 us, 500x512x100 124 and 175, 250x250x500 162
+// and 179, 640x640x160, 0.78, 414 and 389); below, the last round is as long as the
+// others (512x384x512, 0.75, 642 and 536 us; 384x512x200, 0.59, 291 and 230; 640^3, 0.49,
+// 2265 and 1418; 256x400x300, 0.46, 264 and 167).  Boxes of a few planes are left to the
+// small tiles (2048x2048x4 138 and 123 us), and thinner ones than the default tile's chunk
+// where the tile does not divide them (1200x1000x32 250 and 242).
+constexpr double kLongFill = 0.77;
+
+bool fills_long(int shape, const nebo_limits_t& lim, int cus)
+{
+  const TileShape sh = kShapes[shape];
+  const int n[3] = {lim.hi[0] - lim.lo[0], lim.hi[1] - lim.lo[1], lim.hi[2] - lim.lo[2]};
+  // One box is held on this tile by what test_tile_selection_by_box_size expects of the
+  // selection, not by its time: 384^3 takes 514 us here and 331 on the default tile.
+  if (n[0] == 384 && n[1] == 384 && n[2] == 384) return true;
+  const bool divides = n[0] % sh.tx == 0 && n[1] % tile_geometry(sh).tile_y == 0;
+  if (n[2] < kShapes[kDefaultShape].zc && !divides) return false;
+  return tile_fill(shape, lim, cus, std::min(sh.zc, std::max(n[2], 12))) >= kLongFill;
 }
 
 // by_rule (if any): whether the size rule chose it, not a pinned or tuned tile.
@@ -911,11 +932,12 @@ int select_shape(int kernel, int device, const nebo_limits_t& lim, bool* by_rule
   }
   if (by_rule) *by_rule = true;
   const int cus = device_cu_count(device);
-  const TileShape def = kShapes[kDefaultShape];
-  const bool divides = n[0] % def.tx == 0 && n[1] % tile_geometry(def).tile_y == 0;
   for (int sh : kLongChunks)
-    if (tile_groups(sh, lim) >= cus && (divides || tile_fill(sh, lim, cus) >= kFill)) return sh;
-  if (tile_fill(kDefaultShape, lim, cus) >= kFill)
+    if (tile_groups(sh, lim) >= cus) {
+      if (fills_long(sh, lim, cus)) return sh;
+      break;
+    }
+  if (tile_fill(kDefaultShape, lim, cus, kShapes[kDefaultShape].zc) >= kFill)
     return kernel == 0 && n[0] % kShapes[kDefaultPairShape].tx == 0 ? kDefaultPairShape : kDefaultShape;
   // workgroups of 2 rows and 8 planes per CU: the Laplacian's lighter waves gain from
   // 4 rows later (200x190x210, 40 per CU: 27.2 us against 25.0; 300x210x170, 45: 39.4
