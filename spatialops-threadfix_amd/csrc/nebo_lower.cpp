@@ -296,6 +296,16 @@ int assign_limits(const nebo_field_t* lhs, const nebo_expr_t* rhs, int use_ghost
     if (lim->hi[d] - lim->lo[d] <= 0) vol = false;
   }
   *empty = vol ? 0 : 1;
+  // Limits count from the valid region, but reach as far as the LHS's ghosts do: a field
+  // with fewer valid ghosts than ghosts (a scalar assigned to it, or operands with more)
+  // can be covered past its block, which nothing may write.
+  for (int d = 0; d < 3 && vol; ++d) {
+    const long origin = (long)lhs->offset[d] + lhs->valid_minus[d];
+    if (origin + lim->lo[d] < 0 || origin + lim->hi[d] > lhs->glob[d])
+      return set_error(NEBO_ERR_GHOST, ctx,
+                       std::string("The assignment covers cells outside the field's block in the ") + axis[d] +
+                           " direction (fewer valid ghost cells than ghost cells)");
+  }
   return NEBO_OK;
 }
 
