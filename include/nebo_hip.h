@@ -205,7 +205,8 @@ int nebo_device_sync(void);
  * `interior_assign(lhs, rhs)` (use_ghost=0) would cover: calculate_actual_ghost
  * (NeboBasic.h:61-100) + NeboLhs.h:67-88.  Sets *empty when the range has zero
  * volume (no kernel is launched).  Throws the reference's ghost errors as
- * NEBO_ERR_GHOST. */
+ * NEBO_ERR_GHOST, and so limits that reach outside lhs's block, which a field with
+ * fewer valid ghosts than ghosts can have (the reference writes there). */
 int nebo_assign_limits(const nebo_field_t* lhs, const nebo_expr_t* rhs,
                        int use_ghost, nebo_limits_t* limits, int* empty);
 
@@ -253,7 +254,9 @@ int nebo_assign_generic(const nebo_field_t* lhs, const nebo_expr_t* rhs,
  *   nebo_fused_jit_stats: kernels compiled, cache hits, failed compiles;
  *   nebo_fused_source (host only): the kernel source generated for rhs, the
  *   assignment kernel for reduce_op -1, else the NEBO_RED_* reduction kernel
- *   (*needed = bytes with the terminating 0; buf may be NULL). */
+ *   (*needed = bytes with the terminating 0; buf may be NULL).  It knows no box: what
+ *   an assignment's threads, cells and planes are on one, nebo_fused_assign_launch
+ *   tells. */
 int nebo_set_fused_jit(int enable);
 /* Shape of the compiled assignment kernels: threads per block (a multiple of 64
  * in [64, 1024]); tile_x 0 lays a block over consecutive points of the
@@ -291,15 +294,23 @@ int nebo_fused_jit_column(int32_t mode, int32_t waves, int32_t zchunk);
 int nebo_fused_jit_stats(int32_t* compiled, int32_t* cache_hits, int32_t* failures);
 int nebo_fused_source(const nebo_expr_t* rhs, int32_t reduce_op, char* buf, int32_t size,
                       int32_t* needed);
-/* (host only) What nebo_assign would launch for lhs <<= rhs when the tree runs on
- * the compiled column schedule: the kernel source (as nebo_fused_source), its
- * argument struct (args_size bytes at least: 1280), grid and block sizes.
- * NEBO_ERR_UNSUPPORTED when the tree takes another path.  No counterpart in the
+/* (host only) The compiled column-schedule kernel of lhs <<= rhs, also on boxes so small
+ * that nebo_assign runs the tree flattened: the kernel source (as nebo_fused_source),
+ * its argument struct (args_size bytes at least: 1280), grid and block sizes; 8 planes
+ * per block where no GPU is there and nebo_fused_jit_column set none.
+ * NEBO_ERR_UNSUPPORTED when the tree has no such kernel.  No counterpart in the
  * reference: it lets the tests run the generated kernels' address arithmetic on
  * the host and check every access against the fields' allocations. */
 int nebo_fused_column_launch(const nebo_field_t* lhs, const nebo_expr_t* rhs, int use_ghost, char* src,
                              int32_t src_size, int32_t* src_needed, void* args, int32_t args_size,
                              int32_t* grid, int32_t* block);
+/* (host only) The same for the kernel that the generic evaluator compiles and launches for
+ * lhs <<= rhs, whatever its schedule, from the same choice: *column is 1 for the column
+ * schedule, 0 for the flattened plane.  Where no GPU is there, as on one of 256 compute
+ * units. */
+int nebo_fused_assign_launch(const nebo_field_t* lhs, const nebo_expr_t* rhs, int use_ghost, char* src,
+                             int32_t src_size, int32_t* src_needed, void* args, int32_t args_size,
+                             int32_t* grid, int32_t* block, int32_t* column);
 
 /* Which kernel nebo_assign would pick for this tree: 0 generic evaluator,
  * 1 var-coefficient diffusion, 2 Laplacian+Euler, 3 pointwise copy/scale.

@@ -1247,7 +1247,8 @@ double column_steps(const ColumnPlan& cp, int waves, int zc, const int n[3], int
 // was 40 % full), 300^3 428 -> 315, 330x190x410 428 -> 275 (the last of 4 walks of 128
 // planes was a fifth full); div(k grad phi) on 300^3 240 -> 160; filter on 180x150x130
 // 20.0 -> 14.2, 64^3 8.1 -> 4.9.
-bool column_choice(const VmProgram& P, const nebo_limits_t* lim, ColumnPlan* cp, ColumnShape* cs)
+// Without a box (lim null) or compute units (cus 0) the planes are kDefaultColumnZc.
+bool column_choice(const VmProgram& P, const nebo_limits_t* lim, int cus, ColumnPlan* cp, ColumnShape* cs)
 {
   const int mode = g_column.load();
   const bool wide = !lim || lim->hi[0] - lim->lo[0] > 64;
@@ -1258,10 +1259,9 @@ bool column_choice(const VmProgram& P, const nebo_limits_t* lim, ColumnPlan* cp,
     return w ? w : p.pair ? kDefaultPairWaves : kDefaultColumnWaves;
   };
   cs->zc = g_column_zc.load();
-  int device = 0;
-  if (cs->zc == 0 && lim && hipGetDevice(&device) == hipSuccess) {
+  if (cs->zc == 0 && lim && cus > 0) {
     const int n[3] = {lim->hi[0] - lim->lo[0], lim->hi[1] - lim->lo[1], lim->hi[2] - lim->lo[2]};
-    const int simds = 4 * device_cu_count(device);
+    const int simds = 4 * cus;
     double least = 0;
     long total = 0;
     ColumnPlan one = *cp;
@@ -1312,14 +1312,14 @@ bool column_choice(const VmProgram& P, const nebo_limits_t* lim, ColumnPlan* cp,
 // 14.9, 112x96x104 14.4 against 16.0; at 128^3, with 4, 25.8 against 21.3.  With more
 // reads short walks are as fast or faster at every size (div(k grad phi) on 80^3 6.7 us at
 // 4 planes, 8.5 flattened; filter on 100x90x80 6.3 and 9.1).
-bool prefers_flat(const ColumnPlan& cp, const nebo_limits_t& lim)
+bool prefers_flat(const ColumnPlan& cp, const nebo_limits_t& lim, int cus)
 {
   if (g_column_waves.load() || g_column_zc.load()) return false;
-  int reads = 0, device = 0;
+  int reads = 0;
   for (int s = 0; s < kVmMaxLoads; ++s) reads += cp.fam[s] >= 0;
-  if (reads >= 5 * cp.nf || hipGetDevice(&device) != hipSuccess) return false;
+  if (reads >= 5 * cp.nf) return false;
   const int n[3] = {lim.hi[0] - lim.lo[0], lim.hi[1] - lim.lo[1], lim.hi[2] - lim.lo[2]};
-  const int simds = 4 * device_cu_count(device);
+  const int simds = 4 * cus;
   long waves = 0;
   column_steps(cp, cp.pair ? kDefaultPairWaves : kDefaultColumnWaves, 8, n, simds, &waves);
   return waves < simds;
@@ -1412,17 +1412,15 @@ int choose_cells(const VmProgram& P)
 // 9.7 -> 9.4, 256x256x160 50 -> 47; a masked cond 2.8 -> 2.3, 3.4 -> 3.2, 7.6 -> 7.4
 // and (4 cells) 29.4; an upwind transport step (512 threads, 2 cells) 4.6 -> 3.4 on
 // 48x40x36, 8.7 -> 7.7 on 80^3, 14.1 -> 12.5 on 112x96x104.
-int flat_shape(const VmProgram& P, const nebo_limits_t& lim, Shape* sh)
+int flat_shape(const VmProgram& P, const nebo_limits_t& lim, int cus, Shape* sh)
 {
   const int most = choose_cells(P);
-  int device = 0;
   *sh = current_shape();
-  if (g_shape_set.load() || hipGetDevice(&device) != hipSuccess) return most;
+  if (g_shape_set.load()) return most;
   sh->block = 256;
   SlotUse u = slot_use(P);
   for (int m = 0; m < kVmMaxMasks; ++m) u.mused[m] = false;   // bits: next to no bytes
-  const double waves = (double)(lim.hi[0] - lim.lo[0]) * (lim.hi[1] - lim.lo[1]) * (lim.hi[2] - lim.lo[2]) / 64 /
-                       device_cu_count(device);
+  const double waves = (double)(lim.hi[0] - lim.lo[0]) * (lim.hi[1] - lim.lo[1]) * (lim.hi[2] - lim.lo[2]) / 64 / cus;
   const int V = reads_per_thread(u, 4) <= 4 && waves >= 4 * 32 ? 4 : waves >= 2 * 16 ? 2 : 1;
   return std::min(V, most);
 }
@@ -1517,51 +1515,79 @@ int column_args(const nebo_field_t* lhs, const VmProgram& P, const nebo_limits_t
   return NEBO_OK;
 }
 
-int jit_assign(const nebo_field_t* lhs, const VmProgram& P, const nebo_limits_t& lim, void* stream, bool* done)
+// The current device's compute units; 0 where there is no device.
+int current_cus()
 {
-  *done = false;
-  if (!jit_enabled()) return NEBO_OK;
-  Shape sh;
-  const int V = flat_shape(P, lim, &sh);
-  Entry e;
+  int device = 0;
+  if (hipGetDevice(&device) == hipSuccess) return device_cu_count(device);
+  (void)hipGetLastError();
+  return 0;
+}
+
+// What an assignment of P over lim into lhs launches.
+struct AssignLaunch {
+  bool column = false;
   ColumnPlan cp;
   ColumnShape cs;
-  if (column_choice(P, &lim, &cp, &cs) && !prefers_flat(cp, lim)) {
-    int rc = get_kernel_keyed(column_key(P, cp, cs), [&] { return jit_column_source(P, slot_use(P), cp, cs); },
-                              "nebo_fused", &e);
-    if (rc || !e.fn) return rc;
-    JitArgs A;
-    long total = 0;
-    if ((rc = column_args(lhs, P, lim, cp, cs, &A, &total))) return rc;
-    BackendScope bs("compiled kernel, column schedule (" + std::to_string(cs.waves) + " waves per block, " +
-                    std::to_string(cp.RY) + " rows per lane, " + std::to_string(cs.zc) + " planes per block)");
-    if ((rc = emit(stream, CallPtrs{}, replayed_launch(e, A, (unsigned)total, (unsigned)(64 * cs.waves), false))))
-      return rc;
-    *done = true;
-    return NEBO_OK;
+  Shape sh;      // flattened
+  int V = 1;
+  JitArgs args;
+  long grid = 0;
+  int block = 0;
+  std::string key(const VmProgram& P) const { return column ? column_key(P, cp, cs) : structural_key(P, V, sh, -1); }
+  std::string source(const VmProgram& P) const
+  {
+    return column ? jit_column_source(P, slot_use(P), cp, cs) : jit_source(P, V, sh);
   }
-  int rc = get_kernel_keyed(structural_key(P, V, sh, -1), [&] { return jit_source(P, V, sh); }, "nebo_fused", &e);
-  if (rc || !e.fn) return rc;
-  JitArgs A;
-  fill_args(P, lim, V, &A);
+};
+
+int assign_launch(const nebo_field_t* lhs, const VmProgram& P, const nebo_limits_t& lim, int cus, AssignLaunch* L)
+{
+  L->column = column_choice(P, &lim, cus, &L->cp, &L->cs) && !prefers_flat(L->cp, lim, cus);
+  if (L->column) {
+    L->block = 64 * L->cs.waves;
+    return column_args(lhs, P, lim, L->cp, L->cs, &L->args, &L->grid);
+  }
+  L->V = flat_shape(P, lim, cus, &L->sh);
+  fill_args(P, lim, L->V, &L->args);
+  JitArgs& A = L->args;
   A.out = frame_origin(lhs);
   A.oX = lhs->glob[0];
   A.oXY = lhs->glob[0] * lhs->glob[1];
   long ntx;
-  if (sh.tile_x == 0) {
-    ntx = ((long)A.nplane + sh.block - 1) / sh.block;
+  if (L->sh.tile_x == 0) {
+    ntx = ((long)A.nplane + L->sh.block - 1) / L->sh.block;
   } else {
-    const long ty = sh.block / sh.tile_x;
-    ntx = (((long)A.n0 + sh.tile_x - 1) / sh.tile_x) * (((long)A.n1 + ty - 1) / ty);
+    const long ty = L->sh.block / L->sh.tile_x;
+    ntx = (((long)A.n0 + L->sh.tile_x - 1) / L->sh.tile_x) * (((long)A.n1 + ty - 1) / ty);
   }
-  const long total = ntx * A.nzc;
-  if (total >= (1L << 31))
-    return set_error(NEBO_ERR_TOO_LARGE, "Nebo Fused Kernel", "more than 2^31 blocks");
+  L->grid = ntx * A.nzc;
+  L->block = L->sh.block;
+  if (L->grid >= (1L << 31)) return set_error(NEBO_ERR_TOO_LARGE, "Nebo Fused Kernel", "more than 2^31 blocks");
   A.ntx = (int)ntx;
-  A.nblocks = (int)total;
-  BackendScope bs("compiled kernel, " + std::to_string(V) + " z cells per thread (" + std::to_string(sh.block) +
-                  "-thread blocks)");
-  if ((rc = emit(stream, CallPtrs{}, replayed_launch(e, A, (unsigned)total, (unsigned)sh.block, false)))) return rc;
+  A.nblocks = (int)L->grid;
+  return NEBO_OK;
+}
+
+int jit_assign(const nebo_field_t* lhs, const VmProgram& P, const nebo_limits_t& lim, void* stream, bool* done)
+{
+  *done = false;
+  if (!jit_enabled()) return NEBO_OK;
+  AssignLaunch L;
+  int device = 0;
+  int rc = check_hip(hipGetDevice(&device), "Nebo Fused Kernel");
+  if (!rc) rc = assign_launch(lhs, P, lim, device_cu_count(device), &L);
+  if (rc) return rc;
+  Entry e;
+  rc = get_kernel_keyed(L.key(P), [&] { return L.source(P); }, "nebo_fused", &e);
+  if (rc || !e.fn) return rc;
+  BackendScope bs(L.column ? "compiled kernel, column schedule (" + std::to_string(L.cs.waves) +
+                                 " waves per block, " + std::to_string(L.cp.RY) + " rows per lane, " +
+                                 std::to_string(L.cs.zc) + " planes per block)"
+                           : "compiled kernel, " + std::to_string(L.V) + " z cells per thread (" +
+                                 std::to_string(L.sh.block) + "-thread blocks)");
+  if ((rc = emit(stream, CallPtrs{}, replayed_launch(e, L.args, (unsigned)L.grid, (unsigned)L.block, false))))
+    return rc;
   *done = true;
   return NEBO_OK;
 }
@@ -1596,7 +1622,7 @@ std::string jit_source_for(const VmProgram& P, int reduce_op)
   const int V = choose_cells(P);
   ColumnPlan cp;
   ColumnShape cs;
-  if (reduce_op < 0 && column_choice(P, nullptr, &cp, &cs)) return jit_column_source(P, slot_use(P), cp, cs);
+  if (reduce_op < 0 && column_choice(P, nullptr, 0, &cp, &cs)) return jit_column_source(P, slot_use(P), cp, cs);
   return reduce_op < 0 ? jit_source(P, V, current_shape()) : jit_reduce_source(P, V, reduce_op);
 }
 
@@ -1663,29 +1689,26 @@ extern "C" int nebo_fused_jit_stats(int32_t* compiled, int32_t* cache_hits, int3
   return NEBO_OK;
 }
 
-extern "C" int nebo_fused_column_launch(const nebo_field_t* lhs, const nebo_expr_t* rhs, int use_ghost, char* src,
-                                        int32_t src_size, int32_t* src_needed, void* args, int32_t args_size,
-                                        int32_t* grid, int32_t* block)
+namespace {
+
+// The limits and the program of lhs <<= rhs.
+int lower_assignment(const nebo_field_t* lhs, const nebo_expr_t* rhs, int use_ghost, nebo_limits_t* lim,
+                     nebo::VmProgram* P)
 {
   static const char* ctx = "Nebo Fused Kernel";
-  nebo::clear_error();
   if (!lhs || !rhs) return nebo::set_error(NEBO_ERR_INVALID, ctx, "null argument");
-  nebo_limits_t lim;
   int empty = 0;
-  int rc = nebo::assign_limits(lhs, rhs, use_ghost, &lim, &empty);
+  int rc = nebo::assign_limits(lhs, rhs, use_ghost, lim, &empty);
   if (rc) return rc;
   if (empty) return nebo::set_error(NEBO_ERR_UNSUPPORTED, ctx, "empty region: no launch");
-  nebo::VmProgram P;
   int depth = 0;
-  if ((rc = nebo::lower_program(rhs, &P, &depth))) return rc;
-  nebo::ColumnPlan cp;
-  nebo::ColumnShape cs;
-  if (!nebo::column_choice(P, &lim, &cp, &cs))
-    return nebo::set_error(NEBO_ERR_UNSUPPORTED, ctx, "the tree does not run on the column schedule");
-  nebo::JitArgs A;
-  long total = 0;
-  if ((rc = nebo::column_args(lhs, P, lim, cp, cs, &A, &total))) return rc;
-  const std::string s = nebo::jit_column_source(P, nebo::slot_use(P), cp, cs);
+  return nebo::lower_program(rhs, P, &depth);
+}
+
+// A source and an argument struct into the caller's buffers.
+int give_launch(const std::string& s, const nebo::JitArgs& A, char* src, int32_t src_size, int32_t* src_needed,
+                void* args, int32_t args_size)
+{
   if (src_needed) *src_needed = (int32_t)s.size() + 1;
   if (src && src_size > 0) {
     const size_t n = s.size() < (size_t)src_size - 1 ? s.size() : (size_t)src_size - 1;
@@ -1693,11 +1716,56 @@ extern "C" int nebo_fused_column_launch(const nebo_field_t* lhs, const nebo_expr
     src[n] = '\0';
   }
   if (args) {
-    if (args_size < (int32_t)sizeof A) return nebo::set_error(NEBO_ERR_INVALID, ctx, "argument buffer too small");
+    if (args_size < (int32_t)sizeof A)
+      return nebo::set_error(NEBO_ERR_INVALID, "Nebo Fused Kernel", "argument buffer too small");
     std::memcpy(args, &A, sizeof A);
   }
+  return NEBO_OK;
+}
+
+}  // namespace
+
+extern "C" int nebo_fused_column_launch(const nebo_field_t* lhs, const nebo_expr_t* rhs, int use_ghost, char* src,
+                                        int32_t src_size, int32_t* src_needed, void* args, int32_t args_size,
+                                        int32_t* grid, int32_t* block)
+{
+  static const char* ctx = "Nebo Fused Kernel";
+  nebo::clear_error();
+  nebo_limits_t lim;
+  nebo::VmProgram P;
+  int rc = lower_assignment(lhs, rhs, use_ghost, &lim, &P);
+  if (rc) return rc;
+  nebo::ColumnPlan cp;
+  nebo::ColumnShape cs;
+  if (!nebo::column_choice(P, &lim, nebo::current_cus(), &cp, &cs))
+    return nebo::set_error(NEBO_ERR_UNSUPPORTED, ctx, "the tree does not run on the column schedule");
+  nebo::JitArgs A;
+  long total = 0;
+  if ((rc = nebo::column_args(lhs, P, lim, cp, cs, &A, &total))) return rc;
+  rc = give_launch(nebo::jit_column_source(P, nebo::slot_use(P), cp, cs), A, src, src_size, src_needed, args,
+                   args_size);
+  if (rc) return rc;
   if (grid) *grid = (int32_t)total;
   if (block) *block = 64 * cs.waves;
+  return NEBO_OK;
+}
+
+extern "C" int nebo_fused_assign_launch(const nebo_field_t* lhs, const nebo_expr_t* rhs, int use_ghost, char* src,
+                                        int32_t src_size, int32_t* src_needed, void* args, int32_t args_size,
+                                        int32_t* grid, int32_t* block, int32_t* column)
+{
+  nebo::clear_error();
+  nebo_limits_t lim;
+  nebo::VmProgram P;
+  int rc = lower_assignment(lhs, rhs, use_ghost, &lim, &P);
+  if (rc) return rc;
+  const int cus = nebo::current_cus();
+  nebo::AssignLaunch L;
+  if ((rc = nebo::assign_launch(lhs, P, lim, cus ? cus : nebo::device_cu_count(-1), &L))) return rc;
+  if ((rc = give_launch(L.source(P), L.args, src, src_size, src_needed, args, args_size))) return rc;
+  if (grid) *grid = (int32_t)L.grid;
+  if (block) *block = L.block;
+  if (column) *column = L.column ? 1 : 0;
   return NEBO_OK;
 }
 
