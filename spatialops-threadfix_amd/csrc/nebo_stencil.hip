@@ -759,7 +759,7 @@ constexpr int prefetch_planes(const TileShape& sh)
 // 200^3 44.7 against 59.1, 300^3 172 against 182).  An assignment's result may not be
 // read at once, and its nontemporal stores leave that cache to the operands (160^3,
 // three sets of fields in turn: 21.3 us against 30.6).
-constexpr int store_policy(const TileShape& sh) { return sh.variant == 9 ? 0 : 2; }
+constexpr int store_policy(const TileShape& sh, int form = 0);
 constexpr int stacked_waves(const TileShape& sh) { return sh.ty / rows_per_lane(sh); }
 
 // Launch geometry of one tile: rows per tile in y and threads per workgroup
@@ -779,6 +779,18 @@ constexpr Geometry tile_geometry(const TileShape& sh, int kernel = 0)
 // 128^3, a one-wave tile: 18.0 against 23.8).
 constexpr bool writes_images(const TileShape& sh) { return sh.variant < 3 || tile_geometry(sh).threads == kTx; }
 
+constexpr int store_policy(const TileShape& sh, int form)
+{
+  return sh.variant == 9 || (form == 2 && tile_geometry(sh).threads == kTx) ? 0 : 2;
+}
+
+// The pair-column kernel writes no images, which writes_images takes for granted.
+constexpr bool pairs_leave_images(int s = 0)
+{
+  return s >= kNumShapes || ((!pair_columns(kShapes[s]) || !writes_images(kShapes[s])) && pairs_leave_images(s + 1));
+}
+static_assert(pairs_leave_images(), "a pair tile of one wave");
+
 using DivkFn = void (*)(double*, const double*, const double*, Tiles, int, int, nebo_axis_coefs_t, double);
 using LaplFn = void (*)(double*, const double*, Tiles, int, int, nebo_axis_coefs_t, double);
 
@@ -795,7 +807,7 @@ constexpr DivkFn divk_fn()
                                 prefetch_planes(sh)>;
   else if constexpr (sh.variant >= 3)
     return divkgrad_column_kernel<FORM, sh.tx / kTx, stacked_waves(sh), rows_per_lane(sh), sh.zc, sh.variant != 3,
-                                  prefetch_planes(sh), FORM == 2 && tile_geometry(sh).threads == kTx ? 0 : store_policy(sh)>;
+                                  prefetch_planes(sh), store_policy(sh, FORM)>;
   else return divkgrad_staged_kernel<FORM, sh.ty, sh.zc, sh.variant>;
 }
 
@@ -986,7 +998,7 @@ std::string tile_backend_text(const char* kernel, int kind, int shape)
   else
     o << ", column schedule, " << rows_per_lane(sh) << " rows per lane, " << sh.tx / kTx << "x"
       << stacked_waves(sh) << " waves, loads " << prefetch_planes(sh) << " planes ahead"
-      << (store_policy(sh) == 0 ? ", write-back stores" : "");
+      << (store_policy(sh, kind == 1 ? 2 : 0) == 0 ? ", write-back stores" : "");
   return o.str();
 }
 
