@@ -249,9 +249,13 @@ __device__ __forceinline__ double cube_volume(const bool (&has)[3], double size)
 // cells.)  4M particles on 64^3 cells, whose field fits the L2s: 100 us
 // against 175; on 128^3 in random order, where 13M lines miss them (7.5 TB/s from the
 // memory-side cache), 222 against 247, and 87 against 183 where the particles are in
-// cell order.
+// cell order.  AXES are the axes the particles resolve, bit a for axis a, and known to
+// the compiler, since a particle reaches one cell along the others: 1M particles on 64
+// cells of one axis 10.0 us, on 64 x 64 14.8 (15.1 and 19.9 where every axis takes kSpan
+// cells; 12.9 and 23.6 by three nested loops).
 constexpr int kSpan = 3;
 
+template <int AXES>
 __global__ __launch_bounds__(kBlock) void cell_to_particle_kernel(double* __restrict__ dest,
                                                                   const double* __restrict__ src, CellGrid g,
                                                                   Coords pc, const double* __restrict__ psize, long np,
@@ -259,7 +263,8 @@ __global__ __launch_bounds__(kBlock) void cell_to_particle_kernel(double* __rest
 {
   const long p = (long)blockIdx.x * kBlock + threadIdx.x;
   if (p >= np) return;
-  const bool has[3] = {pc.c[0] != nullptr, pc.c[1] != nullptr, pc.c[2] != nullptr};
+  constexpr bool has[3] = {(AXES & 1) != 0, (AXES & 2) != 0, (AXES & 4) != 0};
+  constexpr int span[3] = {has[0] ? kSpan : 1, has[1] ? kSpan : 1, has[2] ? kSpan : 1};
   PRange r;
   if (!particle_range(g, has, load_particle(pc, psize, p), &r)) {
     if (skipped) atomicAdd(skipped, 1);
@@ -279,11 +284,11 @@ __global__ __launch_bounds__(kBlock) void cell_to_particle_kernel(double* __rest
     };
     const double* cell0 = src + (g.origin + r.lo[0] * g.stride[0] + r.lo[1] * g.stride[1] + r.lo[2] * g.stride[2]);
     double w[3][kSpan];
-    bool fast = nx <= kSpan && ny <= kSpan && nz <= kSpan && divisor_safe(vol);
+    bool fast = nx <= span[0] && ny <= span[1] && nz <= span[2] && divisor_safe(vol);
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll
-      for (int i = 0; i < kSpan; ++i) {
+      for (int i = 0; i < span[a]; ++i) {
         w[a][i] = part(a, r.lo[a] + i);
         // an overlap of zero gives a quotient of zero (of either sign: the sum starts at
         // +0, so it never shows); three others multiply to a safe dividend
@@ -292,24 +297,24 @@ __global__ __launch_bounds__(kBlock) void cell_to_particle_kernel(double* __rest
     if (fast) {
       double xy[kSpan][kSpan];
 #pragma unroll
-      for (int j = 0; j < kSpan; ++j)
+      for (int j = 0; j < span[1]; ++j)
 #pragma unroll
-        for (int i = 0; i < kSpan; ++i) xy[j][i] = w[0][i] * w[1][j];
+        for (int i = 0; i < span[0]; ++i) xy[j][i] = w[0][i] * w[1][j];
 #pragma unroll
-      for (int k = 0; k < kSpan; ++k) {
+      for (int k = 0; k < span[2]; ++k) {
         if (k < nz) {
           double v[kSpan][kSpan];
 #pragma unroll
-          for (int j = 0; j < kSpan; ++j)
+          for (int j = 0; j < span[1]; ++j)
 #pragma unroll
-            for (int i = 0; i < kSpan; ++i) {
+            for (int i = 0; i < span[0]; ++i) {
               v[j][i] = 0.0;
               if (j < ny && i < nx) v[j][i] = cell0[i * g.stride[0] + j * g.stride[1] + k * g.stride[2]];
             }
 #pragma unroll
-          for (int j = 0; j < kSpan; ++j)
+          for (int j = 0; j < span[1]; ++j)
 #pragma unroll
-            for (int i = 0; i < kSpan; ++i)
+            for (int i = 0; i < span[0]; ++i)
               if (j < ny && i < nx) acc += v[j][i] * quotient(xy[j][i] * w[2][k], vol, rvol);
         }
       }
@@ -970,7 +975,11 @@ extern "C" int nebo_cell_to_particle(double* dest, const nebo_field_t* src, cons
   const CellGrid g = make_grid(src, *geom);
   const Coords pc{{px, py, pz}};
   const long blocks = (np + kBlock - 1) / kBlock;
-  hipLaunchKernelGGL(cell_to_particle_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, (hipStream_t)stream,
+  using Gather = void (*)(double*, const double*, CellGrid, Coords, const double*, long, int*);
+  static const Gather gather[8] = {cell_to_particle_kernel<0>, cell_to_particle_kernel<1>, cell_to_particle_kernel<2>,
+                                   cell_to_particle_kernel<3>, cell_to_particle_kernel<4>, cell_to_particle_kernel<5>,
+                                   cell_to_particle_kernel<6>, cell_to_particle_kernel<7>};
+  hipLaunchKernelGGL(gather[(px ? 1 : 0) | (py ? 2 : 0) | (pz ? 4 : 0)], dim3((unsigned)blocks), dim3(kBlock), 0, (hipStream_t)stream,
                      dest, static_cast<const double*>(src->values), g, pc, psize, (long)np, skipped);
   return check_hip(hipGetLastError(), ctx);
 }

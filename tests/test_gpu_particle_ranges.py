@@ -51,3 +51,24 @@ def test_ranges_past_32_bits(axes):
     orc.particle_to_cell(cells, src, *coords, size, geom)
     torch.cuda.synchronize()
     assert np.array_equal(cells.gpu.cpu().numpy(), cells.host, equal_nan=True)
+
+
+@pytest.mark.parametrize("mask", range(8))
+def test_every_set_of_resolved_axes(mask):
+    """Axes the particles do not resolve, on a window of several cells along them."""
+    n = (9, 8, 7)
+    L = nh.Layout.build(n, 1)
+    rng = np.random.default_rng(40 + mask)
+    m = 2000
+    size = rng.uniform(0.2, 4.0, m)
+    coords = [rng.uniform(-1.0, n[a] + 1.0, m) if mask >> a & 1 else None for a in range(3)]
+    cells = nh.Field.from_numpy(L, rng.standard_normal(L.npts), where="both")
+    op = P.CellToParticle(*GEOM)
+    op.set_coordinate_information(*[None if c is None else dev(c) for c in coords], dev(size))
+    skipped = torch.zeros(1, dtype=torch.int32, device="cuda:0")
+    out = op.apply_to_field(cells, torch.full((m,), 9.0, dtype=torch.float64, device="cuda:0"), skipped=skipped)
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy(), orc.cell_to_particle(cells, *coords, size, GEOM, m))
+    # skipped: a cell or more below the window (face -1.0) on some axis
+    low = [(c - size * 0.5 + 1.0) / 1.0 for c in coords if c is not None]
+    assert skipped.item() == (int(np.any([t <= -1.0 for t in low], axis=0).sum()) if low else 0)
