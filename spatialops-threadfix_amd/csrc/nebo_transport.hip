@@ -26,6 +26,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 
 namespace nebo {
@@ -510,8 +511,14 @@ struct StagePlan {
 // direct one; its z chunk applies to either).  us per stage of 8 steps' worth of
 // launches in a hipGraph, stage 2 and its transpose:
 //  1. the 128 x 8 tile with loads 1 plane ahead and the longest chunk (512 .. 64
-//     planes) that gives every CU a workgroup, where the box fills two thirds of the
-//     cells its rounds of workgroups hold (256^3: 197 and 326);
+//     planes) that gives every CU a workgroup, where the box holds two thirds of the
+//     cells its rounds of workgroups walk (256^3: 197 and 326; 512x512x300 829 and 1433
+//     against 1043 and 1596 on the tiles of 2., 512x512x64 193 and 316 against 242 and
+//     358; 384x512x200, 0.59 in two rounds, 614 and 996 against 545 and 838); the
+//     transpose in more than one round only where they are as full as those tiles
+//     (512x384x512, 0.75, 2191 against 2109; 1200x1000x32, 0.92, 852 and 801; 1024x512x40
+//     438 and 457); boxes of fewer than 10 planes leave it (512x512x8 31 and 45 against 27
+//     and 38);
 //  2. boxes that give a CU 28 waves of 2 rows x 8 planes: one-wave tiles of 4 rows
 //     and 8 planes (200^3: 111 and 177 against 132 and 256 direct);
 //  3. the transpose on smaller boxes, down to 2.5 such waves: one-wave tiles of 2 rows
@@ -545,9 +552,11 @@ StagePlan stage_plan(const nebo_field_t* f, bool transpose)
     const int tx = kLanes * kColW, ty = kColRY * kColNW;
     const double cells = (double)n[0] * n[1] * n[2];
     for (int c : {512, 256, 128, 64}) {
-      const long g = groups(tx, ty, c);
+      const long g = groups(tx, ty, c), rounds = (g + cus - 1) / cus;
       if (g < cus) continue;
-      if (cells >= 0.66 * (double)((g + cus - 1) / cus * cus) * tx * ty * c) {
+      const double fill = cells / ((double)rounds * cus * tx * ty * std::min(c, n[2]));
+      const double small_fill = cells / ((double)groups(kLanes, 4, 8) * kLanes * 4 * 8);
+      if (n[2] >= 10 && fill >= (transpose && rounds > 1 ? 0.98 * small_fill : 0.66)) {
         P.sched = 3;   // loads 1 plane ahead: 1388 us per stage at 512^3 on MI355X, 2 planes 1413, direct 1797
         auto_zc = c;
       }
