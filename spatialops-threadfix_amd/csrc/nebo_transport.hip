@@ -318,8 +318,17 @@ __global__ __launch_bounds__(1024) void transport_adjoint_kernel(
   double ac = a[i], sc = s[i], kc = k[i];
   AdjFace zlo = adj_face(a[i - XY], ac, s[i - XY], sc, k[i - XY], kc, uz[i], cz);
   for (int z = z0; z < z1; ++z, i += XY) {
-    const double az = a[i + XY], szp = s[i + XY], kzp = k[i + XY], gc = gk[i];
-    const double ain = STAGE == 3 ? 0.0 : acc_in[i];   // stage 3 reads no acc_in
+    const double az = a[i + XY], szp = s[i + XY], kzp = k[i + XY];
+    // The cell's own g_k and acc_in (none in stage 3) come with the plane, but after its
+    // faces in stage 2, which has both to read and write: with them the compiler kept to
+    // 96 registers by issuing the plane's loads in groups (stage 2 on 64^3 8.9 -> 7.4 us,
+    // 256x256x64 with direct loads 124 -> 95, 256^3 501 -> 380).
+    double gc = 0.0, ain = 0.0;
+    auto load_own = [&]() __attribute__((always_inline)) {
+      gc = gk[i];
+      if constexpr (STAGE != 3) ain = acc_in[i];
+    };
+    if constexpr (STAGE != 2) load_own();
     const AdjFace xlo = adj_face(a[i - 1], ac, s[i - 1], sc, k[i - 1], kc, ux[i], cx);
     const AdjFace xhi = adj_face(ac, a[i + 1], sc, s[i + 1], kc, k[i + 1], ux[i + 1], cx);
     const AdjFace ylo = adj_face(a[i - X], ac, s[i - X], sc, k[i - X], kc, uy[i], cy);
@@ -331,6 +340,7 @@ __global__ __launch_bounds__(1024) void transport_adjoint_kernel(
     const double v = STAGE == 1 ? ain + Xv : cs * Xv;
     out[i] = v;
     store_images(&out[i], x, y, z, B.n, X, XY, v);
+    if constexpr (STAGE == 2) load_own();
     if constexpr (STAGE == 3) acc_out[i] = (1.0 / 3.0) * ac;
     else if constexpr (STAGE == 2) acc_out[i] = ain + 0.75 * ac;
     gk[i] = gc + cdt * ((ex.B + ey.B) + ez.B);
@@ -522,14 +532,15 @@ struct StagePlan {
 //  2. boxes that give a CU 28 waves of 2 rows x 8 planes: one-wave tiles of 4 rows
 //     and 8 planes (200^3: 111 and 177 against 132 and 256 direct);
 //  3. the transpose on smaller boxes, down to 2.5 such waves: one-wave tiles of 2 rows
-//     and 8 planes, 4 planes below 6 waves (160^3: 78 against 127 direct, 112x96x80:
-//     18.6 against 22.3); the stage, with fewer fields, is as fast on direct loads
-//     there (160^3 44.3 against 42.1, 112x96x80 13.5 against 12.3);
+//     and 8 planes, 4 planes below 6 waves (160^3: 78 against 104 direct, 128^3 34.8 and
+//     34.5, 112x96x80 18.9 and 17.6, 90x80x70 15.8 and 17.1); the stage, with fewer
+//     fields, is as fast on direct loads there (160^3 44.3 against 42.1, 112x96x80 13.5
+//     against 12.3);
 //  4. direct loads: a wave per 4 planes of one row, two rows and 16 planes per
 //     workgroup; where that leaves a CU fewer than 8 waves, per 2 planes, one row per
-//     workgroup (64^3: 5.0 and 8.7 against 22.9 and 28.6 with 16 planes per wave, whose
+//     workgroup (64^3: 5.5 and 7.4 against 22.9 and 28.6 with 16 planes per wave, whose
 //     chain of planes set the time); and workgroups of 4 rows and 2 planes where even
-//     those leave CUs without one (32^3: 3.7 and 5.5 against 23.1 and 26.8).
+//     those leave CUs without one (32^3: 4.0 and 4.7 against 23.1 and 26.8).
 // One-wave tiles write back, for the next pass to read (trajectory gradients at 200^3
 // 4832 us against 4960, 300^3 14981 against 15251), but those of 2 rows store
 // nontemporally where the transpose's 11 fields do not fit the 256 MB memory-side cache
