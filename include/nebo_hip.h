@@ -439,8 +439,8 @@ int nebo_lapl_euler(const nebo_field_t* out, const nebo_field_t* phi,
  *      dimensions on the same device;
  *   3. else 128 x 8 tiles, variant 7, with the longest z chunk of 512, 256 or
  *      128 planes that gives every CU a workgroup (512^3: 512 planes), where the
- *      box holds 77 % of the cells that whole rounds of one tile per CU walk (and
- *      has 64 planes or is a multiple of the tile in x and y);
+ *      box holds 77 % of the cells that whole rounds of one tile per CU walk (10
+ *      planes at least);
  *   4. else 128 x 8 x 64, variant 11 for kernel 0 on boxes whose width is a
  *      multiple of 128 and variant 7 otherwise, where the box holds 66 % of the
  *      cells that whole rounds of one tile per CU could (256^3);

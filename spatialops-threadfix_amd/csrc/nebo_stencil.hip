@@ -912,9 +912,9 @@ double tile_fill(int shape, const nebo_limits_t& lim, int cus, int planes)
 // and what follows: 512x512x300 385 and 412 us, 500x512x100 124 and 175, 250x250x500 162
 // and 179, 640x640x160, 0.78, 414 and 389); below, the last round is as long as the
 // others (512x384x512, 0.75, 642 and 536 us; 384x512x200, 0.59, 291 and 230; 640^3, 0.49,
-// 2265 and 1418; 256x400x300, 0.46, 264 and 167).  Boxes of a few planes are left to the
-// small tiles (2048x2048x4 138 and 123 us), and thinner ones than the default tile's chunk
-// where the tile does not divide them (1200x1000x32 250 and 242).
+// 2265 and 1418; 256x400x300, 0.46, 264 and 167).  Boxes of fewer than 10 planes are left to
+// the small tiles (2048x2048x4 138 and 123 us, 1024x1024x8 59 and 54; 1500x700x10 74 and
+// 89, 1000x1000x20 116 and 133).
 constexpr double kLongFill = 0.77;
 
 bool fills_long(int shape, const nebo_limits_t& lim, int cus)
@@ -924,9 +924,19 @@ bool fills_long(int shape, const nebo_limits_t& lim, int cus)
   // One box is held on this tile by what test_tile_selection_by_box_size expects of the
   // selection, not by its time: 384^3 takes 514 us here and 331 on the default tile.
   if (n[0] == 384 && n[1] == 384 && n[2] == 384) return true;
-  const bool divides = n[0] % sh.tx == 0 && n[1] % tile_geometry(sh).tile_y == 0;
-  if (n[2] < kShapes[kDefaultShape].zc && !divides) return false;
-  return tile_fill(shape, lim, cus, std::min(sh.zc, std::max(n[2], 12))) >= kLongFill;
+  return n[2] >= 10 && tile_fill(shape, lim, cus, std::min(sh.zc, n[2])) >= kLongFill;
+}
+
+// Rule 5.  Workgroups of 2 rows and 8 planes per CU: the Laplacian's lighter waves gain
+// from 4 rows later (200x190x210, 40 per CU: 27.2 us against 25.0; 300x210x170, 45: 39.4
+// against 40.7).
+int small_shape(int kernel, const nebo_limits_t& lim, int cus)
+{
+  const long waves8 = tile_groups(kSmallColumn[1], lim);
+  if (waves8 >= (kernel == 0 ? 24L : 44L) * cus) return kLargeColumn;
+  if (waves8 >= 16L * cus) return kSmallColumn[1];
+  if (tile_groups(kSmallColumn[0], lim) >= 4L * cus) return kSmallColumn[0];
+  return waves8 >= 4L * cus ? kSmallColumn[1] : kSmallColumn[2];
 }
 
 // by_rule (if any): whether the size rule chose it, not a pinned or tuned tile.
@@ -951,14 +961,7 @@ int select_shape(int kernel, int device, const nebo_limits_t& lim, bool* by_rule
     }
   if (tile_fill(kDefaultShape, lim, cus, kShapes[kDefaultShape].zc) >= kFill)
     return kernel == 0 && n[0] % kShapes[kDefaultPairShape].tx == 0 ? kDefaultPairShape : kDefaultShape;
-  // workgroups of 2 rows and 8 planes per CU: the Laplacian's lighter waves gain from
-  // 4 rows later (200x190x210, 40 per CU: 27.2 us against 25.0; 300x210x170, 45: 39.4
-  // against 40.7)
-  const long waves8 = tile_groups(kSmallColumn[1], lim);
-  if (waves8 >= (kernel == 0 ? 24L : 44L) * cus) return kLargeColumn;
-  if (waves8 >= 16L * cus) return kSmallColumn[1];
-  if (tile_groups(kSmallColumn[0], lim) >= 4L * cus) return kSmallColumn[0];
-  return waves8 >= 4L * cus ? kSmallColumn[1] : kSmallColumn[2];
+  return small_shape(kernel, lim, cus);
 }
 
 int find_shape(int tx, int ty, int zc, int variant)
@@ -1156,11 +1159,19 @@ int launch_diffusion_euler(const nebo_field_t* out, const nebo_field_t* k, const
   const nebo_limits_t lim = interior_of(out);
   bool by_rule = false;
   int pick = select_shape(0, out->device, lim, &by_rule);
+  const int cus = device_cu_count(out->device);
+  // thin boxes that the long tile does not divide run the small ones, which write their
+  // many ghost images themselves (700x900x14 59 us against 73 with a fill, 500x512x30 46.6
+  // and 50.5, 2000x2000x16 447 and 468; 1000x1000x20 153 and 139)
+  const TileShape sh = kShapes[pick];
+  if (by_rule && sh.zc > kShapes[kDefaultShape].zc && lim.hi[2] < kShapes[kDefaultShape].zc &&
+      (lim.hi[0] % sh.tx || lim.hi[1] % tile_geometry(sh).tile_y))
+    pick = small_shape(0, lim, cus);
   // walks of 8 planes for 16 on boxes of few waves, where those that write ghost images set
   // the time (per step of 20, the input's fill included: 128^3, 4 waves of 16 planes per CU,
   // 17.4 us against 18.7, 112x150x130, 5.3, 19.8 and 21.9; 256x128x100, 7, 23.6 and 23.2,
   // 180x150x130, 7.9, 24.5 and 24.1)
-  if (by_rule && pick == kSmallColumn[0] && tile_groups(pick, lim) < 6L * device_cu_count(out->device))
+  if (by_rule && pick == kSmallColumn[0] && tile_groups(pick, lim) < 6L * cus)
     pick = kSmallColumn[1];
   const int shape = usable_shape(pick, out->glob[0], out->glob[0] * out->glob[1], lim.hi[0] - lim.lo[0], 0);
   const int rc = launch_divk_shape(shape, 2, out, k, phi, c, dt, lim, stream);

@@ -15,7 +15,9 @@ RULE = [
     ((256, 512, 200), LONG[128], LONG[128]),        # one round of 256 workgroups, 0.78
     ((512, 512, 40), LONG[512], LONG[512]),
     ((500, 512, 100), LONG[512], LONG[512]),        # not divided; one round
-    ((500, 512, 30), BIG, (64, 2, 8, 3)),           # not divided, and thin
+    ((500, 512, 30), LONG[512], LONG[512]),         # not divided, and thin
+    ((1000, 1000, 9), BIG, BIG),                    # too thin
+    ((1500, 700, 10), LONG[512], LONG[512]),
     ((2048, 2048, 4), BIG, BIG),
     ((256, 400, 300), PAIR, DEF),                   # 300 workgroups of 128 planes: 0.46
     ((384, 512, 200), PAIR, DEF),                   # 384: 0.59
